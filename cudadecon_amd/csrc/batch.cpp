@@ -182,6 +182,7 @@ void Batch::build_groups() {
     std::map<ZKey, const float2*> ztw;
     std::map<int, long> ytot;
     std::map<ZKey, long> ztot;
+    std::map<ZKey, bool> zbuf;
     for (int p = P1.p0; p < P1.p1; ++p) {
       const int i = order[p];
       const RLEngine& e = *engines[i];
@@ -189,7 +190,7 @@ void Batch::build_groups() {
       float2* S = a_spec.as<float2>() + soff[i];
       {
         const long L = col_tile_cols(F.ny), nt = (F.nxh + L - 1) / L;
-        ColSeg sg{S, F.nxh, F.pitch, (long)F.ny * F.pitch, nt, ytot[F.ny]};
+        ColSeg sg{S, F.nxh, F.pitch, (long)F.ny * F.pitch, nt, ytot[F.ny], e.otf.params(e.table, 1.0).sup};
         ys[F.ny].push_back(sg);
         ytot[F.ny] += (long)F.nz * nt;
         ytw[F.ny] = F.twy.as<float2>();
@@ -198,6 +199,7 @@ void Batch::build_groups() {
         const long L = col_tile_cols(F.nz), nt = (F.nxh + L - 1) / L;
         const OtfParams op = e.otf.params(e.table, 1.0 / (double)F.nvox);
         const ZKey key{F.nz, op.ra != 0};
+        zbuf[key] = (ztot[key] == 0 || zbuf[key]) && z_ragged_buf(F.nz, (long)F.ny * F.pitch);
         ZSeg sg{S, F.nxh, (long)F.ny * F.pitch, F.pitch, nt, F.ny, ztot[key], op};
         zs[key].push_back(sg);
         ztot[key] += (long)F.ny * nt;
@@ -219,6 +221,7 @@ void Batch::build_groups() {
       ColGroup g;
       g.len = kv.first.first;
       g.ra = kv.first.second;
+      g.buf = zbuf[kv.first];
       g.nseg = (int)kv.second.size();
       g.total = ztot[kv.first];
       g.tw = ztw[kv.first];
@@ -293,7 +296,8 @@ void Batch::enqueue_partition(const Partition& P, hipStream_t st, int iters, hip
         launch_col_ragged(g.len, 0, st, g.segs.as<ColSeg>(), g.nseg, g.total, g.tw, grid_cap);
       CDN_HIP(hipEventRecord(mark, st));
       for (const ColGroup& g : P.zg)
-        launch_z_ragged(g.len, st, g.segs.as<ZSeg>(), g.nseg, g.total, f, g.tw, grid_cap, g.ra);
+        launch_z_ragged(g.len, st, g.segs.as<ZSeg>(), g.nseg, g.total, f, g.tw, grid_cap, g.ra,
+                        g.buf);
       CDN_HIP(hipEventRecord(mark, st));
       for (const ColGroup& g : P.yg)
         launch_col_ragged(g.len, 1, st, g.segs.as<ColSeg>(), g.nseg, g.total, g.tw, grid_cap);

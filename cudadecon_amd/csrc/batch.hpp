@@ -58,6 +58,7 @@ struct Batch {
   struct ColGroup {
     int len = 0, nseg = 0;
     bool ra = false;  // z groups: every table rotationally averaged
+    bool buf = true;  // z groups: launch_z_ragged's buf
     long total = 0;
     const float2* tw = nullptr;
     DevBuf segs;

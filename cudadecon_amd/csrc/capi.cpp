@@ -531,10 +531,10 @@ int cudaDecon_filter(float* vol, int nx, int ny, int nz, const float* otf, int o
       float2* S = ds.as<float2>();
       launch_x_r2c(nx, st, dv.as<float>(), nullptr, nullptr, nullptr, XIN_PLAIN, S, (long)ny * nz, F.pitch,
                    F.twx.as<float2>());
-      F.col(st, S, 1, false);
-      launch_z_filter(nz, st, S, F.nxh, (long)ny * F.pitch, F.pitch, ny, conj, D.params(T, 1.0 / (double)F.nvox),
-                      F.twz.as<float2>());
-      F.col(st, S, 1, true);
+      const OtfParams op = D.params(T, 1.0 / (double)F.nvox);
+      F.col(st, S, 1, false, op.sup);
+      launch_z_filter(nz, st, S, F.nxh, (long)ny * F.pitch, F.pitch, ny, conj, op, F.twz.as<float2>());
+      F.col(st, S, 1, true, op.sup);
       launch_x_c2r(nx, st, S, dv.as<float>(), (long)ny * nz, F.pitch, F.twx.as<float2>());
       copy_to_host(st, vol, dv.p, sizeof(float) * F.nvox);
     } catch (...) {

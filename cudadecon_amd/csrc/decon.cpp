@@ -108,9 +108,9 @@ void Fft3::setup(int x, int y, int z, hipStream_t st, DevRegion* region) {
   fft_prepare_cols(nz, nxh);
 }
 
-void Fft3::col(hipStream_t st, float2* S, int axis, bool inverse) const {
+void Fft3::col(hipStream_t st, float2* S, int axis, bool inverse, const OtfSupport& sup) const {
   if (axis == 1)
-    launch_col_fft(ny, inverse, st, S, nxh, pitch, (long)ny * pitch, nz, twy.as<float2>());
+    launch_col_fft(ny, inverse, st, S, nxh, pitch, (long)ny * pitch, nz, twy.as<float2>(), sup);
   else
     launch_col_fft(nz, inverse, st, S, nxh, (long)ny * pitch, pitch, ny, twz.as<float2>());
 }
@@ -195,6 +195,12 @@ OtfParams OtfDev::params(const OtfTable& t, double inv_n) const {
   p.kyscale = ks[1];
   p.kzscale = ks[2];
   p.inv_n = (float)inv_n;
+  // points with kr >= nr - 1 are zero (z filter); the bound is taken 1e-4
+  // larger, far above the rounding of kr, so it never cuts a nonzero one
+  p.sup = kNoSupport;
+  const double rmax = (t.nxotf - 1) * 1.0001;
+  if (ra && ks[0] > 0.f && ks[1] > 1e-6f && ks[0] < 1e6f && ks[1] < 1e6f)
+    p.sup = OtfSupport{(float)(rmax * rmax), ks[0], (float)(1.0 / ks[1])};
   return p;
 }
 
@@ -333,13 +339,13 @@ void RLEngine::iterate(int n, int k0, bool seeded, hipStream_t st, double* lambd
     for (int f = 0; f < 2; ++f) {
       // the y transforms see the stacks as nz nstacks slabs
       launch_col_fft(fft.ny, 0, st, S, fft.nxh, fft.pitch, (long)fft.ny * fft.pitch, (long)fft.nz * nstacks,
-                     fft.twy.as<float2>());
+                     fft.twy.as<float2>(), op.sup);
       mark(PASS_YFWD);
       launch_z_filter(fft.nz, st, S, fft.nxh, (long)fft.ny * fft.pitch, fft.pitch, fft.ny, f, op, twz, nstacks,
                       fft.nspec);
       mark(PASS_ZFILT);
       launch_col_fft(fft.ny, 1, st, S, fft.nxh, fft.pitch, (long)fft.ny * fft.pitch, (long)fft.nz * nstacks,
-                     fft.twy.as<float2>());
+                     fft.twy.as<float2>(), op.sup);
       mark(PASS_YINV);
       if (f == 0) {
         launch_x_lrcore(fft.nx, st, S, raw.as<float>(), rows, fft.pitch, twx, eps);

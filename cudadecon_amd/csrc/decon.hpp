@@ -79,7 +79,8 @@ struct Fft3 {
   void setup(int x, int y, int z, hipStream_t st, DevRegion* region = nullptr);
   void r2c(hipStream_t st, const float* in, float2* S) const;   // unnormalised
   void c2r(hipStream_t st, float2* S, float* out) const;        // unnormalised, consumes S
-  void col(hipStream_t st, float2* S, int axis, bool inverse) const;  // axis 1 = y, 2 = z
+  // axis 1 = y, 2 = z; sup: of the OTF of the z filter between the y transforms
+  void col(hipStream_t st, float2* S, int axis, bool inverse, const OtfSupport& sup = kNoSupport) const;
 };
 
 struct OtfDev {

@@ -264,34 +264,44 @@ void fft_prepare_cols(int len, long ncols) {
 }
 
 void launch_col_fft(int len, int inverse, hipStream_t st, float2* S, long ncols, long line_stride,
-                    long outer_stride, long n_outer, const float2* tw) {
+                    long outer_stride, long n_outer, const float2* tw, const OtfSupport& sup) {
   FftVariant tv;
   const bool tuned = col_variant(len, ncols, &tv);
   const CShape cs = c_shape(len, tuned ? tv.cols : -1, tuned ? tv.col_tpt : -1);
   long ntiles = (ncols + cs.L - 1) / cs.L;
   const unsigned grid = grid1(ntiles * n_outer);
-  void* args[] = {&S, &ncols, &line_stride, &outer_stride, &ntiles, &tw};
+  OtfSupport sp = sup;
+  // a slab's rows by 32-bit offsets (always the case for y transforms: at
+  // most 16384 rows of 8208 columns)
+  const bool buf = (double)len * (double)line_stride * 8.0 < 2147483648.0;
+  if (!buf && sp.r2 >= 0.f) fail("launch_col_fft: support bound on a slab of 2 GiB or more");
+  void* args[] = {&S, &ncols, &line_stride, &outer_stride, &ntiles, &sp, &tw};
+  const JitKernel jk = inverse ? (buf ? JK_COL_I : JK_COL_IW) : (buf ? JK_COL_F : JK_COL_FW);
   if (tuned) {
-    jit_launch(len, inverse ? JK_COL_I : JK_COL_F, grid, cs.THREADS, st, args, tv);
+    jit_launch(len, jk, grid, cs.THREADS, st, args, tv);
   } else {
     switch (len) {
-#define CDN_CASE(N)                                                                                            \
-  case N:                                                                                                      \
-    if (inverse)                                                                                               \
-      hipLaunchKernelGGL((k_col<N, true>), dim3(grid), dim3(cs.THREADS), 0, st, S, ncols, line_stride,         \
-                         outer_stride, ntiles, tw);                                                            \
-    else                                                                                                       \
-      hipLaunchKernelGGL((k_col<N, false>), dim3(grid), dim3(cs.THREADS), 0, st, S, ncols, line_stride,        \
-                         outer_stride, ntiles, tw);                                                            \
-    break;
+#define CDN_CASE(N)                                                                                                  \
+  case N: {                                                                                                          \
+    auto* k = inverse ? (buf ? k_col<N, true, true> : k_col<N, true, false>)                                         \
+                      : (buf ? k_col<N, false, true> : k_col<N, false, false>);                                      \
+    hipLaunchKernelGGL(k, dim3(grid), dim3(cs.THREADS), 0, st, S, ncols, line_stride, outer_stride, ntiles, sp, tw); \
+    break;                                                                                                           \
+  }
       CDN_FFT_LENGTHS(CDN_CASE)
 #undef CDN_CASE
       default:
-        jit_launch(len, inverse ? JK_COL_I : JK_COL_F, grid, cs.THREADS, st, args);
+        jit_launch(len, jk, grid, cs.THREADS, st, args);
     }
   }
   CDN_HIP(hipGetLastError());
 }
+
+// the z filter's buffers (TPT planes each) take 32-bit offsets
+static bool z_buf(const CShape& cs, long line_stride) {
+  return (double)cs.TPT * (double)line_stride * 8.0 < 2147483648.0;
+}
+bool z_ragged_buf(int nz, long line_stride) { return z_buf(c_shape(nz), line_stride); }
 
 void launch_z_filter(int nz, hipStream_t st, float2* S, long ncols, long line_stride, long outer_stride, long ny,
                      int conj, const OtfParams& otf, const float2* tw, int nstacks, long stack_stride) {
@@ -304,20 +314,20 @@ void launch_z_filter(int nz, hipStream_t st, float2* S, long ncols, long line_st
   OtfParams op = otf;
   void* args[] = {&S, &ncols, &line_stride, &outer_stride, &ntiles, &ny, &stack_stride, &conj, &op, &tw};
   // the averaged-table kind for a rotationally averaged OTF
-  const JitKernel jk = op.ra ? JK_Z_FILTER_RA : JK_Z_FILTER;
+  const bool ra = op.ra != 0, buf = z_buf(cs, line_stride);
+  const JitKernel jk = ra ? (buf ? JK_Z_FILTER_RA : JK_Z_FILTER_RA_W) : (buf ? JK_Z_FILTER : JK_Z_FILTER_W);
   if (tuned) {
     jit_launch(nz, jk, grid, cs.THREADS, st, args, tv);
   } else {
     switch (nz) {
-#define CDN_CASE(N)                                                                                          \
-  case N:                                                                                                    \
-    if (op.ra)                                                                                               \
-      hipLaunchKernelGGL((k_z_filter<N, ZF_RA>), dim3(grid), dim3(cs.THREADS), 0, st, S, ncols, line_stride, \
-                         outer_stride, ntiles, ny, stack_stride, conj, op, tw);                              \
-    else                                                                                                     \
-      hipLaunchKernelGGL((k_z_filter<N, ZF_ANY>), dim3(grid), dim3(cs.THREADS), 0, st, S, ncols,             \
-                         line_stride, outer_stride, ntiles, ny, stack_stride, conj, op, tw);                 \
-    break;
+#define CDN_CASE(N)                                                                                             \
+  case N: {                                                                                                     \
+    auto* k = ra ? (buf ? k_z_filter<N, ZF_RA, true> : k_z_filter<N, ZF_RA, false>)                             \
+                 : (buf ? k_z_filter<N, ZF_ANY, true> : k_z_filter<N, ZF_ANY, false>);                          \
+    hipLaunchKernelGGL(k, dim3(grid), dim3(cs.THREADS), 0, st, S, ncols, line_stride, outer_stride, ntiles, ny, \
+                       stack_stride, conj, op, tw);                                                             \
+    break;                                                                                                      \
+  }
       CDN_FFT_LENGTHS(CDN_CASE)
 #undef CDN_CASE
       default:
@@ -379,38 +389,36 @@ void launch_col_ragged(int len, int inverse, hipStream_t st, const ColSeg* segs,
   CDN_HIP(hipGetLastError());
 }
 
-// the kernel instance for (persistent, kind)
+// the kernel instance for (persistent, kind, buffer addressing); stacks that
+// need 64-bit addresses fill the GPU one item per workgroup
 template <int N>
-static void z_ragged_n(bool pers, bool ra, unsigned grid, unsigned threads, hipStream_t st, const ZSeg* segs,
-                       int nseg, long total, int conj, const float2* tw) {
-  if (pers && ra)
-    hipLaunchKernelGGL((k_z_ragged<N, true, ZF_RA>), dim3(grid), dim3(threads), 0, st, segs, nseg, total, conj, tw);
-  else if (pers)
-    hipLaunchKernelGGL((k_z_ragged<N, true, ZF_ANY>), dim3(grid), dim3(threads), 0, st, segs, nseg, total, conj, tw);
-  else if (ra)
-    hipLaunchKernelGGL((k_z_ragged<N, false, ZF_RA>), dim3(grid), dim3(threads), 0, st, segs, nseg, total, conj, tw);
-  else
-    hipLaunchKernelGGL((k_z_ragged<N, false, ZF_ANY>), dim3(grid), dim3(threads), 0, st, segs, nseg, total, conj,
-                       tw);
+static auto z_ragged_n(bool pers, bool ra, bool buf) {
+  if (!buf) return ra ? k_z_ragged<N, false, ZF_RA, false> : k_z_ragged<N, false, ZF_ANY, false>;
+  return pers ? (ra ? k_z_ragged<N, true, ZF_RA> : k_z_ragged<N, true, ZF_ANY>)
+              : (ra ? k_z_ragged<N, false, ZF_RA> : k_z_ragged<N, false, ZF_ANY>);
 }
 
 void launch_z_ragged(int nz, hipStream_t st, const ZSeg* segs, int nseg, long total, int conj, const float2* tw,
-                     long grid_cap, bool ra) {
+                     long grid_cap, bool ra, bool buf) {
   if (total <= 0) return;
   const CShape cs = c_shape(nz);
-  const unsigned grid = ragged_grid(total, grid_cap);
+  const unsigned grid = ragged_grid(total, buf ? grid_cap : 0);
   const bool pers = grid < total;
   void* args[] = {&segs, &nseg, &total, &conj, &tw};
   switch (nz) {
-#define CDN_CASE(N)                                                                    \
-  case N:                                                                              \
-    z_ragged_n<N>(pers, ra, grid, cs.THREADS, st, segs, nseg, total, conj, tw);     \
-    break;
+#define CDN_CASE(N)                                                                                        \
+  case N: {                                                                                                \
+    auto* k = z_ragged_n<N>(pers, ra, buf);                                                                \
+    hipLaunchKernelGGL(k, dim3(grid), dim3(cs.THREADS), 0, st, segs, nseg, total, conj, tw);               \
+    break;                                                                                                 \
+  }
     CDN_FFT_LENGTHS(CDN_CASE)
 #undef CDN_CASE
-    default:
-      jit_launch(nz, pers ? (ra ? JK_Z_RAGGED_P_RA : JK_Z_RAGGED_P) : (ra ? JK_Z_RAGGED_RA : JK_Z_RAGGED), grid,
-                 cs.THREADS, st, args);
+    default: {
+      const JitKernel b[4] = {JK_Z_RAGGED, JK_Z_RAGGED_P, JK_Z_RAGGED_RA, JK_Z_RAGGED_P_RA};
+      const JitKernel w[2] = {JK_Z_RAGGED_W, JK_Z_RAGGED_RA_W};
+      jit_launch(nz, buf ? b[2 * ra + pers] : w[ra], grid, cs.THREADS, st, args);
+    }
   }
   CDN_HIP(hipGetLastError());
 }

@@ -69,10 +69,15 @@ struct BuiltinShapesOnly {
 };
 void fft_clear_variants();
 
+// a bound that no column exceeds
+constexpr OtfSupport kNoSupport{-1.f, 0.f, 0.f};
+
 // Column FFT (forward or inverse) over `len` points at element stride
-// line_stride, for columns [0, ncols) of each of n_outer slabs.
+// line_stride, for columns [0, ncols) of each of n_outer slabs.  sup: for the
+// y transforms around a z filter, the support of its OTF (the rows outside it
+// are not stored by the forward and taken as zero by the inverse transform).
 void launch_col_fft(int len, int inverse, hipStream_t st, float2* S, long ncols, long line_stride,
-                    long outer_stride, long n_outer, const float2* tw);
+                    long outer_stride, long n_outer, const float2* tw, const OtfSupport& sup = kNoSupport);
 // z forward -> x H (or conj H) / N -> z inverse; slab index = ky, for
 // nstacks spectra stack_stride complex elements apart.
 void launch_z_filter(int nz, hipStream_t st, float2* S, long ncols, long line_stride, long outer_stride,
@@ -92,6 +97,9 @@ void launch_col_ragged(int len, int inverse, hipStream_t st, const ColSeg* segs,
 // ra: every segment's OTF is rotationally averaged (the kernel kind the
 // one-stack z filter uses for such a table)
 void launch_z_ragged(int nz, hipStream_t st, const ZSeg* segs, int nseg, long total, int conj, const float2* tw,
-                     long grid_cap = 0, bool ra = false);
+                     long grid_cap = 0, bool ra = false, bool buf = true);
+// whether a stack's z filter can address its planes (line_stride apart) by
+// 32-bit offsets: buf above, for every segment of the launch
+bool z_ragged_buf(int nz, long line_stride);
 
 }  // namespace cdn

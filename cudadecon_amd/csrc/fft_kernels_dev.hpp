@@ -644,35 +644,106 @@ __device__ __forceinline__ void col_line(float2 (&v)[CCfg<N>::E], float2* lds, i
   }
 }
 
-// tile lb (slab-major) of a column pass; lds as declared by the kernel
-template <int N, bool INV>
+// The largest |ky| at which the OTF can be nonzero in column kx = c (-1:
+// none; never increasing with c).  The z filter multiplies the rows beyond it
+// by zero: the forward y transform does not store them, the z filter neither
+// reads nor writes them, and the inverse y transform takes them as zero.
+// With data and PSF sampled alike the table ends at the Nyquist radius and
+// 21% of the (kx, ky) plane lies outside.  At 256 x 1024 x 1024: z filter
+// 0.451 -> 0.354 ms, y forward 0.381 -> 0.352, y inverse 0.382 -> 0.357,
+// iteration 4.53 -> 4.23 ms; at 96 x 2048 x 2048 7.95 -> 7.40 ms, at
+// 768 x 384 x 96 0.72 -> 0.64 (with SlabBuf below).
+// The kernels must agree on the bound, so no product here may be fused into a
+// multiply-add in one and not in another.
+__device__ __forceinline__ int support_ky(const OtfSupport& s, long c) {
+#pragma clang fp contract(off)
+  if (s.r2 < 0.f) return 0x7fffffff;
+  const float kx = (float)c * s.ksx;
+  const float d = s.r2 - kx * kx;
+  return d >= 0.f ? (int)(sqrtf(d) * s.iky) + 1 : -1;
+}
+
+// One slab of a spectrum as a buffer resource (32-bit byte offsets, scalar
+// row offsets): a thread keeps one offset for all its loads and stores
+// instead of a 64-bit address each, and a load at kNoRow returns zero without
+// touching memory, so skipping rows needs no branches.  The inverse y pass
+// with a branch per skipped row needs 75 registers at 1024 points, which
+// leaves one workgroup per CU instead of two (0.393 ms, every row read 0.382,
+// this form 0.357).  Registers of the y transforms: 64 to 2048 points 60-92
+// -> 56-81, of the z filters 92-142 -> 84-126 at 64 to 192 points.
+constexpr int kNoRow = -1;  // outside every slab
+typedef unsigned u2v __attribute__((ext_vector_type(2)));
+struct SlabBuf {
+  __amdgpu_buffer_rsrc_t rs;
+  __device__ __forceinline__ SlabBuf(float2* slab, int bytes)
+      : rs(__builtin_amdgcn_make_buffer_rsrc(slab, 0, bytes, 0x00020000)) {}
+  template <bool NT> __device__ __forceinline__ float2 load(int off, int row_off) const {
+    const u2v t = __builtin_amdgcn_raw_buffer_load_b64(rs, off, row_off, NT ? 2 : 0);
+    return make_float2(__uint_as_float(t.x), __uint_as_float(t.y));
+  }
+  template <bool NT> __device__ __forceinline__ void store(int off, int row_off, float2 v) const {
+    u2v t;
+    t.x = __float_as_uint(v.x);
+    t.y = __float_as_uint(v.y);
+    __builtin_amdgcn_raw_buffer_store_b64(t, rs, off, row_off, NT ? 2 : 0);
+  }
+};
+
+// The 256-point forward transform keeps plain addresses: with buffers the
+// compiler fuses the other product of two terms of its radix-16 stages into
+// multiply-adds, and results move by rounding.  Every other built-in length
+// gives the same bits either way (all lengths, directions and filter kinds
+// compared).
+constexpr bool col_buf(int N, bool inv) { return N != 256 || inv; }
+
+// tile lb (slab-major) of a column pass; lds as declared by the kernel.  sup:
+// for the y transforms around a z filter, its OTF's support.  BUF: a
+// slab (N rows) spans less than 2^31 bytes.
+template <int N, bool INV, bool BUF>
 __device__ __forceinline__ void col_tile(float2* lds, float2* __restrict__ S, long ncols, long line_stride,
-                                         long outer_stride, long ntiles, long lb, const float2* __restrict__ tw) {
+                                         long outer_stride, long ntiles, long lb, const OtfSupport& sup,
+                                         const float2* __restrict__ tw) {
   using C = CCfg<N>;
   const int tid = threadIdx.x;
   const int l = tid % C::L, p = tid / C::L;
   const long outer = lb / ntiles, tile = lb - outer * ntiles;
   const long c = tile * C::L + l;
   const bool valid = c < ncols;
-  float2* base = S + outer * outer_stride + c;
   float2 v[C::E];
+  if constexpr (BUF && col_buf(N, INV)) {
+    const int ls8 = (int)line_stride * 8;
+    const SlabBuf slab(S + outer * outer_stride, N * ls8);
+    const int off = valid ? p * ls8 + (int)c * 8 : kNoRow;
+    // row i holds ky = i or i - N; the z filter reads and writes none beyond lim
+    const int lim = support_ky(sup, c);
+    auto live = [&](int i) { return min(i, N - i) <= lim ? off : kNoRow; };
 #pragma unroll
-  for (int m = 0; m < C::E; ++m)
-    v[m] = valid ? ld_stream<NTCL>(base + (long)(p + m * C::TPT) * line_stride) : make_float2(0.f, 0.f);
-  col_line<N, INV>(v, lds, l, p, tw);
-  if (valid) {
+    for (int m = 0; m < C::E; ++m)
+      v[m] = slab.template load<NTCL>(INV ? live(p + m * C::TPT) : off, m * C::TPT * ls8);
+    col_line<N, INV>(v, lds, l, p, tw);
 #pragma unroll
-    for (int m = 0; m < C::E; ++m) st_stream<NTCS>(base + (long)(p + m * C::TPT) * line_stride, v[m]);
+    for (int m = 0; m < C::E; ++m)
+      slab.template store<NTCS>(INV ? off : live(p + m * C::TPT), m * C::TPT * ls8, v[m]);
+  } else {
+    float2* base = S + outer * outer_stride + c;
+#pragma unroll
+    for (int m = 0; m < C::E; ++m)
+      v[m] = valid ? ld_stream<NTCL>(base + (long)(p + m * C::TPT) * line_stride) : make_float2(0.f, 0.f);
+    col_line<N, INV>(v, lds, l, p, tw);
+    if (valid) {
+#pragma unroll
+      for (int m = 0; m < C::E; ++m) st_stream<NTCS>(base + (long)(p + m * C::TPT) * line_stride, v[m]);
+    }
   }
 }
 
-template <int N, bool INV>
+template <int N, bool INV, bool BUF = true>
 __global__ void __launch_bounds__(CCfg<N>::THREADS)
-    k_col(float2* __restrict__ S, long ncols, long line_stride, long outer_stride, long ntiles,
+    k_col(float2* __restrict__ S, long ncols, long line_stride, long outer_stride, long ntiles, OtfSupport sup,
           const float2* __restrict__ tw) {
   __shared__ float2 lds[CCfg<N>::LDS];
-  col_tile<N, INV>(lds, S, ncols, line_stride, outer_stride, ntiles,
-                   xcd_logical_block<CCfg<N>::L>(blockIdx.x, gridDim.x), tw);
+  col_tile<N, INV, BUF>(lds, S, ncols, line_stride, outer_stride, ntiles,
+                        xcd_logical_block<CCfg<N>::L>(blockIdx.x, gridDim.x), sup, tw);
 }
 
 // segment holding work item `it`: the last whose item0 <= it (segs[0].item0 = 0)
@@ -703,7 +774,8 @@ __global__ void __launch_bounds__(CCfg<N>::THREADS)
   do {
     const long lb = xcd_logical_block<CCfg<N>::L>(it, total);
     const ColSeg& g = segs[find_seg(segs, nseg, lb)];
-    col_tile<N, INV>(lds, g.S, g.ncols, g.line_stride, g.outer_stride, g.ntiles, lb - g.item0, tw);
+    col_tile<N, INV, true>(lds, g.S, g.ncols, g.line_stride, g.outer_stride, g.ntiles, lb - g.item0, g.sup,
+                     tw);
     if constexpr (!PERSIST) break;
     __syncthreads();  // the next item's exchanges reuse lds
     it += gridDim.x;
@@ -764,25 +836,28 @@ template <int N, int KIND> struct ZRows {
 
 // filter_kernel / filterConj_kernel (src/RLgpuImpl.cu:331-350) with the OTF
 // value computed on the fly as in dev_otfinterpolate (src/RLgpuImpl.cu:228-329)
-template <int N, int KIND = ZF_ANY>
+// BUF: TPT rows (planes) span less than 2^31 bytes (z_buf).
+template <int N, int KIND = ZF_ANY, bool BUF = true>
 __global__ void __launch_bounds__(CCfg<N>::THREADS) __attribute__((amdgpu_waves_per_eu(zf_waves(N, KIND))))
     k_z_filter(float2* __restrict__ S, long ncols, long line_stride, long outer_stride, long ntiles, long ny,
                long stack_stride, int conj, OtfParams otf, const float2* __restrict__ tw) {
   using C = CCfg<N>;
   constexpr int RS = ZRows<N, KIND>::R;
   constexpr int PER = RS > 0 ? (RS * N + C::THREADS - 1) / C::THREADS : 1;
-  constexpr bool ZRA = KIND == ZF_RA;
+  constexpr bool ZRA = KIND == ZF_RA, ZBUF = BUF;
   __shared__ float2 lds[C::LDS];
   __shared__ float2 otf_rows[RS > 0 ? RS * N : 1];
   const long lb = xcd_logical_block<C::L>(blockIdx.x, gridDim.x);
+  do {
 #include "zf_tile_body.inc"
+  } while (false);
 }
 
 // The z filter of every stack whose z length is N, stacks of different shapes
 // and OTFs in one launch (ZSeg per stack); items and PERSIST as k_col_ragged.
 // KIND as k_z_filter's (ZF_RA: every segment's table is rotationally
 // averaged), so that each stack runs the code its one-stack engine runs.
-template <int N, bool PERSIST, int KIND = ZF_ANY>
+template <int N, bool PERSIST, int KIND = ZF_ANY, bool BUF = true>
 __global__ void __launch_bounds__(CCfg<N>::THREADS) __attribute__((amdgpu_waves_per_eu(zf_waves(N, KIND))))
     k_z_ragged(const ZSeg* __restrict__ segs, int nseg, long total, int conj, const float2* __restrict__ tw) {
   using C = CCfg<N>;
@@ -798,10 +873,10 @@ __global__ void __launch_bounds__(CCfg<N>::THREADS) __attribute__((amdgpu_waves_
     const long ncols = g->ncols, line_stride = g->line_stride, outer_stride = g->outer_stride;
     const long ntiles = g->ntiles, ny = g->ny, stack_stride = 0, lb = gi - g->item0;
     const OtfParams& otf = g->otf;
-    constexpr bool ZRA = KIND == ZF_RA;
-    {
+    constexpr bool ZRA = KIND == ZF_RA, ZBUF = BUF;
+    do {
 #include "zf_tile_body.inc"
-    }
+    } while (false);
     if constexpr (!PERSIST) break;
     __syncthreads();  // the next item's exchanges and staged rows reuse lds
     it += gridDim.x;

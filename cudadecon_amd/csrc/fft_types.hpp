@@ -26,12 +26,21 @@ struct Otf3d {
   int nxotf, nyotf, nzotf;
 };
 
+// The half-spectrum points where a rotationally averaged OTF can be nonzero:
+// kr = |(kx, ky)| below the last radial sample.  r2 < 0: no bound.
+struct OtfSupport {
+  float r2;   // the squared radius, a little above the table's
+  float ksx;  // radius per kx column
+  float iky;  // ky rows per unit of radius
+};
+
 struct OtfParams {
   int ra;  // 1: rotationally averaged (RaOtf), 0: 3-D table (Otf3d)
   RaOtf ra_tab;
   Otf3d tab3;
   float kxscale, kyscale, kzscale;
   float inv_n;  // 1 / (nx ny nz): the filter's normalisation
+  OtfSupport sup;
 };
 
 // One stack's share of a column pass that spans stacks of different shapes
@@ -41,6 +50,7 @@ struct OtfParams {
 struct ColSeg {
   float2* S;
   long ncols, line_stride, outer_stride, ntiles, item0;
+  OtfSupport sup;
 };
 // The same for the z filter (slabs are ky rows; the stack's own OTF).
 struct ZSeg {

@@ -35,7 +35,10 @@ const char* const kExpr[JK_COUNT] = {"cdn::k_x_r2c<%d, false>",   "cdn::k_x_c2r<
                                      "cdn::k_z_ragged<%d, false>", "cdn::k_col_ragged<%d, false, true>",
                                      "cdn::k_col_ragged<%d, true, true>", "cdn::k_z_ragged<%d, true>",
                                      "cdn::k_z_filter<%d, 1>",    "cdn::k_z_ragged<%d, false, 1>",
-                                     "cdn::k_z_ragged<%d, true, 1>"};
+                                     "cdn::k_z_ragged<%d, true, 1>",
+                                     "cdn::k_col<%d, false, false>", "cdn::k_col<%d, true, false>",
+                                     "cdn::k_z_filter<%d, 0, false>", "cdn::k_z_filter<%d, 1, false>",
+                                     "cdn::k_z_ragged<%d, false, 0, false>", "cdn::k_z_ragged<%d, false, 1, false>"};
 const char* const kOpts[] = {"--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature",
                              "-Xclang", "-packed-fp32-ops"};
 

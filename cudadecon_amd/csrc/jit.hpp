@@ -27,6 +27,13 @@ enum JitKernel {
   JK_Z_FILTER_RA,
   JK_Z_RAGGED_RA,
   JK_Z_RAGGED_P_RA,
+  // _W: slabs too large for 32-bit offsets
+  JK_COL_FW,
+  JK_COL_IW,
+  JK_Z_FILTER_W,
+  JK_Z_FILTER_RA_W,
+  JK_Z_RAGGED_W,
+  JK_Z_RAGGED_RA_W,
   JK_COUNT
 };
 

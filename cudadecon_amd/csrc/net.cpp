@@ -9,8 +9,11 @@
 namespace cdn {
 namespace {
 
-constexpr int WG_CHUNKS = 64;       // weight-gradient partial rows (3x3x3 layers, x27 taps)
-constexpr int WG_CHUNKS_IN1 = 512;  // first layer
+// weight-gradient partial rows, one per workgroup: two or more workgroups per
+// CU, and a quarter of that where a row is 4 times as long (32 <-> 64 channels)
+constexpr int WG_CHUNKS = 512;
+constexpr int wg_chunks(int l) { return NET_CIN[l] * NET_COUT[l] > 1024 ? WG_CHUNKS / 2 : WG_CHUNKS; }
+constexpr int WG_CHUNKS_IN1 = 1024;  // first layer
 constexpr int CS_BLOCKS = 256;      // bias-gradient partial rows
 
 struct SplitMix {
@@ -120,7 +123,7 @@ void WarmNet::geometry(int nb, int nz, int ny, int nx, bool training) {
     g1.ensure(h * n1 * 16);
     hpart.ensure(sizeof(float) * 18 * (size_t)net_head_blocks(L1));
     cpart.ensure(sizeof(float) * 64 * CS_BLOCKS);
-    wpart.ensure(sizeof(float) * std::max(27L * 64 * 32 * WG_CHUNKS, 27L * 16 * WG_CHUNKS_IN1));
+    wpart.ensure(sizeof(float) * std::max(27L * 64 * 32 * wg_chunks(2), 27L * 16 * WG_CHUNKS_IN1));
     loss.ensure(sizeof(float) * 4);
   }
 }
@@ -170,8 +173,8 @@ void WarmNet::backward(hipStream_t st, const float* raw, const float* tgt, float
   net_head_reduce(st, hpart.as<float>(), hb, 1.0 / (double)vox(L1), g, head_off, loss_slot);
 
   auto wgrad = [&](int l, const bf16_t* in, const bf16_t* gr, const Vol& v) {
-    net_wgrad(st, NET_CIN[l], NET_COUT[l], in, gr, v, WG_CHUNKS, wpart.as<float>());
-    net_reduce_rows(st, wpart.as<float>(), WG_CHUNKS, 27L * NET_CIN[l] * NET_COUT[l], g + w_off[l]);
+    const int rows = net_wgrad(st, NET_CIN[l], NET_COUT[l], in, gr, v, wg_chunks(l), wpart.as<float>());
+    net_reduce_rows(st, wpart.as<float>(), rows, 27L * NET_CIN[l] * NET_COUT[l], g + w_off[l]);
     net_chan_sum(st, NET_COUT[l], gr, vox(v), CS_BLOCKS, cpart.as<float>());
     net_reduce_rows(st, cpart.as<float>(), CS_BLOCKS, NET_COUT[l], g + b_off[l]);
   };
@@ -193,8 +196,8 @@ void WarmNet::backward(hipStream_t st, const float* raw, const float* tgt, float
   net_conv(st, 32, 16, false, g2.as<bf16_t>(), wb[1].as<bf16_t>(), nullptr, gP1.as<bf16_t>(), L2);
   // conv1 (u -> e1); e1 also feeds the head directly
   net_grad_enc(st, 16, e1.as<bf16_t>(), nullptr, dO, wh, gP1.as<bf16_t>(), g1.as<bf16_t>(), L1);
-  net_wgrad_in1(st, raw, inv_s.as<float>(), g1.as<bf16_t>(), L1, WG_CHUNKS_IN1, wpart.as<float>());
-  net_reduce_rows(st, wpart.as<float>(), WG_CHUNKS_IN1, 27L * 16, g + w_off[0]);
+  const int rows1 = net_wgrad_in1(st, raw, inv_s.as<float>(), g1.as<bf16_t>(), L1, WG_CHUNKS_IN1, wpart.as<float>());
+  net_reduce_rows(st, wpart.as<float>(), rows1, 27L * 16, g + w_off[0]);
   net_chan_sum(st, 16, g1.as<bf16_t>(), vox(L1), CS_BLOCKS, cpart.as<float>());
   net_reduce_rows(st, cpart.as<float>(), CS_BLOCKS, 16, g + b_off[0]);
 }

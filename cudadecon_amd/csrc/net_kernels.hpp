@@ -41,8 +41,9 @@ void net_grad_enc(hipStream_t st, int c, const bf16_t* e, const bf16_t* skip, co
 void net_grad_dec(hipStream_t st, int c, const bf16_t* d, const bf16_t* fine, const float* dout, const float* wh,
                   bf16_t* dpre, Vol coarse);
 void net_chan_sum(hipStream_t st, int c, const bf16_t* t, long nvox, int blocks, float* part);
-void net_wgrad(hipStream_t st, int cin, int cout, const bf16_t* in, const bf16_t* g, Vol v, int G, float* part);
-void net_wgrad_in1(hipStream_t st, const float* raw, const float* inv_s, const bf16_t* g, Vol v, int G, float* part);
+// weight gradients in at most G partial rows of 27 cin cout; returns how many
+int net_wgrad(hipStream_t st, int cin, int cout, const bf16_t* in, const bf16_t* g, Vol v, int G, float* part);
+int net_wgrad_in1(hipStream_t st, const float* raw, const float* inv_s, const bf16_t* g, Vol v, int G, float* part);
 void net_reduce_rows(hipStream_t st, const float* part, int rows, long cols, float* out);
 int net_sum_blocks(int nb);
 void net_inv_scale(hipStream_t st, const float* raw, Vol v, double* part, float* inv_s);

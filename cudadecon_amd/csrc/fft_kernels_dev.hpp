@@ -249,39 +249,86 @@ template <int N> struct CCfg {
   static constexpr int LDS = HALF ? (N * L + 1) / 2 : N * L;  // float2 elements
 };
 
+// A piece of a volume or spectrum as a buffer resource (32-bit byte offsets,
+// scalar row offsets): a thread keeps one offset for all its loads and stores
+// instead of a 64-bit address each, and a load at kNoRow returns zero without
+// touching memory, so skipping rows needs no branches.  The inverse y pass
+// with a branch per skipped row needs 75 registers at 1024 points, which
+// leaves one workgroup per CU instead of two (0.393 ms, every row read 0.382,
+// this form 0.357).  Registers of the y transforms: 64 to 2048 points 60-92
+// -> 56-81, of the z filters 92-142 -> 84-126 at 64 to 192 points.
+// Loads past the end return zero and stores there do nothing.
+constexpr int kNoRow = -1;  // past every end
+typedef unsigned u2v __attribute__((ext_vector_type(2)));
+struct SlabBuf {
+  __amdgpu_buffer_rsrc_t rs;
+  __device__ __forceinline__ SlabBuf(const void* slab, int bytes)
+      : rs(__builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(slab), 0, bytes, 0x00020000)) {}
+  template <bool NT> __device__ __forceinline__ float2 load(int off, int row_off) const {
+    const u2v t = __builtin_amdgcn_raw_buffer_load_b64(rs, off, row_off, NT ? 2 : 0);
+    return make_float2(__uint_as_float(t.x), __uint_as_float(t.y));
+  }
+  template <bool NT> __device__ __forceinline__ void store(int off, int row_off, float2 v) const {
+    u2v t;
+    t.x = __float_as_uint(v.x);
+    t.y = __float_as_uint(v.y);
+    __builtin_amdgcn_raw_buffer_store_b64(t, rs, off, row_off, NT ? 2 : 0);
+  }
+  template <bool NT> __device__ __forceinline__ float load1(int off, int row_off) const {
+    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, off, row_off, NT ? 2 : 0));
+  }
+};
+
+
 // ---------------------------------------------------------------------------
 // x passes.  Thread p of a line holds v[m] = z[p + m TPT] with z = a + i b
 // for the two real rows r0, r0+1 packed into one complex line.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ float load_y(int mode, const float* __restrict__ X, const float* __restrict__ Xp,
-                                        float* __restrict__ Y, float lam, long idx) {
-  if (mode == XIN_PRED) {
-    const float x = X[idx], xp = Xp[idx];
-    float y = x + lam * (x - xp);
-    y = y > 0.f ? y : 0.f;
-    Y[idx] = y;
-    return y;
-  }
-  if (mode == XIN_SEED) return Y[idx];
-  return X[idx];
-}
-
 __device__ __forceinline__ float2 shfl2(float2 v, int src) {
   return make_float2(__shfl(v.x, src, 64), __shfl(v.y, src, 64));
 }
 
+// Where an x pass reads and writes the half spectra of its row pair (A: first
+// row, B: second; zero past the last row): element p + m STEP of both rows, or
+// nothing (on false).  RowsPtr by address; RowsBuf through a buffer over the
+// workgroup's rows.
+template <int STEP> struct RowsPtr {
+  float2* S;  // element p of the first row
+  long pitch;
+  bool v0, v1;
+  __device__ __forceinline__ void load(int m, bool on, float2& A, float2& B) const {
+    A = on && v0 ? ld_stream<NTX>(S + m * STEP) : make_float2(0.f, 0.f);
+    B = on && v1 ? ld_stream<NTX>(S + pitch + m * STEP) : make_float2(0.f, 0.f);
+  }
+  __device__ __forceinline__ void store(int m, bool on, float2 A, float2 B) const {
+    if (!on) return;
+    if (v0) st_stream<NTX>(S + m * STEP, A);
+    if (v1) st_stream<NTX>(S + pitch + m * STEP, B);
+  }
+};
+template <int STEP> struct RowsBuf {
+  SlabBuf b;
+  int off, pitch8;  // bytes: of element p of the first row, per row
+  __device__ __forceinline__ void load(int m, bool on, float2& A, float2& B) const {
+    A = b.template load<NTX>(on ? off : kNoRow, m * STEP * 8);
+    B = b.template load<NTX>(on ? off : kNoRow, m * STEP * 8 + pitch8);
+  }
+  __device__ __forceinline__ void store(int m, bool on, float2 A, float2 B) const {
+    b.template store<NTX>(on ? off : kNoRow, m * STEP * 8, A);
+    b.template store<NTX>(on ? off : kNoRow, m * STEP * 8 + pitch8, B);
+  }
+};
+
 // Half spectra A (row r0) and B (row r0+1) from the packed transform Z:
 // A[k] = (Z[k] + conj Z[N-k]) / 2, B[k] = (Z[k] - conj Z[N-k]) / (2i).
-template <int N, int K = XK_PLAIN>
-__device__ __forceinline__ void split_store(float2 (&v)[(XCfg<N, K>::E)], float2* line, int p,
-                                            float2* __restrict__ S, long r0, long pitch, bool v0, bool v1) {
+template <int N, int K = XK_PLAIN, class Rows>
+__device__ __forceinline__ void split_store(float2 (&v)[(XCfg<N, K>::E)], float2* line, int p, const Rows& rows) {
   using C = XCfg<N, K>;
   constexpr int E = C::E, TPT = C::TPT;
-  auto put = [&](int k, float2 zk, float2 zn) {
+  auto put = [&](int m, bool on, float2 zk, float2 zn) {
     const float2 A = make_float2(0.5f * (zk.x + zn.x), 0.5f * (zk.y - zn.y));
     const float2 D = make_float2(0.5f * (zk.x - zn.x), 0.5f * (zk.y + zn.y));
-    if (v0) st_stream<NTX>(S + r0 * pitch + k, A);
-    if (v1) st_stream<NTX>(S + (r0 + 1) * pitch + k, make_float2(D.y, -D.x));
+    rows.store(m, on, A, make_float2(D.y, -D.x));
   };
   if constexpr (C::SHUFFLE) {
     // element N-k of k = p + m TPT sits in lane (TPT-p) % TPT of this line,
@@ -292,7 +339,7 @@ __device__ __forceinline__ void split_store(float2 (&v)[(XCfg<N, K>::E)], float2
     for (int m = 0; m <= E / 2; ++m) {
       const float2 t = shfl2(v[E - 1 - m], src);
       const float2 zn = (p == 0) ? v[(E - m) % E] : t;
-      if (m < E / 2 || p == 0) put(p + m * TPT, v[m], zn);
+      put(m, m < E / 2 || p == 0, v[m], zn);
     }
   } else {
 #pragma unroll
@@ -301,21 +348,20 @@ __device__ __forceinline__ void split_store(float2 (&v)[(XCfg<N, K>::E)], float2
 #pragma unroll
     for (int e = 0; e < C::EH; ++e) {
       const int k = p + e * TPT;
-      if (k <= N / 2) put(k, line[k], line[k == 0 ? 0 : N - k]);
+      if (k <= N / 2) put(e, true, line[k], line[k == 0 ? 0 : N - k]);
     }
   }
 }
 
 // Packed line Z = A + i B (Hermitian extension of both rows; imaginary parts
 // of the kx = 0 and kx = N/2 bins ignored) into v.
-template <int N, int K = XK_PLAIN>
-__device__ __forceinline__ void merge_load(float2 (&v)[(XCfg<N, K>::E)], float2* line, int p,
-                                           const float2* __restrict__ S, long r0, long pitch, bool v0, bool v1) {
+template <int N, int K = XK_PLAIN, class Rows>
+__device__ __forceinline__ void merge_load(float2 (&v)[(XCfg<N, K>::E)], float2* line, int p, const Rows& rows) {
   using C = XCfg<N, K>;
   constexpr int E = C::E, TPT = C::TPT;
-  auto ld = [&](int k, float2& A, float2& B) {
-    A = v0 ? ld_stream<NTX>(S + r0 * pitch + k) : make_float2(0.f, 0.f);
-    B = v1 ? ld_stream<NTX>(S + (r0 + 1) * pitch + k) : make_float2(0.f, 0.f);
+  auto ld = [&](int m, bool on, float2& A, float2& B) {
+    const int k = p + m * TPT;
+    rows.load(m, on, A, B);
     if (k == 0 || 2 * k == N) {
       A.y = 0.f;
       B.y = 0.f;
@@ -324,10 +370,8 @@ __device__ __forceinline__ void merge_load(float2 (&v)[(XCfg<N, K>::E)], float2*
   if constexpr (C::SHUFFLE) {
     float2 A[E / 2 + 1], B[E / 2 + 1];
 #pragma unroll
-    for (int m = 0; m < E / 2; ++m) ld(p + m * TPT, A[m], B[m]);
-    A[E / 2] = make_float2(0.f, 0.f);
-    B[E / 2] = make_float2(0.f, 0.f);
-    if (p == 0) ld(N / 2, A[E / 2], B[E / 2]);
+    for (int m = 0; m < E / 2; ++m) ld(m, true, A[m], B[m]);
+    ld(E / 2, p == 0, A[E / 2], B[E / 2]);
 #pragma unroll
     for (int m = 0; m < E / 2; ++m) v[m] = make_float2(A[m].x - B[m].y, A[m].y + B[m].x);
     const int lane = threadIdx.x & 63;
@@ -351,7 +395,7 @@ __device__ __forceinline__ void merge_load(float2 (&v)[(XCfg<N, K>::E)], float2*
       const int k = p + e * TPT;
       if (k <= N / 2) {
         float2 A, B;
-        ld(k, A, B);
+        ld(e, true, A, B);
         line[k] = make_float2(A.x - B.y, A.y + B.x);
         if (k != 0 && 2 * k != N) line[N - k] = make_float2(A.x + B.y, B.x - A.y);
       }
@@ -433,7 +477,7 @@ __global__ void __launch_bounds__((XCfg<N, XK_R2C>::THREADS))
   for (int m = 0; m < C::E; ++m) v[m] = make_float2(a[m], b[m]);
   fft_line<N, C::TPT, 1, false>(v, line, p, tw);
   __syncthreads();
-  split_store<N, XK_R2C>(v, line, p, S, r0, pitch, v0, v1);
+  split_store<N, XK_R2C>(v, line, p, RowsPtr<C::TPT>{S + r0 * pitch + p, pitch, v0, v1});
 }
 
 template <int N>
@@ -448,7 +492,7 @@ __global__ void __launch_bounds__(XCfg<N>::THREADS)
   const bool v0 = r0 < rows, v1 = r0 + 1 < rows;
   float2* line = lds + l * C::LS;
   float2 v[C::E];
-  merge_load<N>(v, line, p, S, r0, pitch, v0, v1);
+  merge_load<N>(v, line, p, RowsPtr<C::TPT>{const_cast<float2*>(S) + r0 * pitch + p, pitch, v0, v1});
   fft_line<N, C::TPT, 1, true>(v, line, p, tw);
 #pragma unroll
   for (int m = 0; m < C::E; ++m) {
@@ -467,6 +511,16 @@ __device__ __forceinline__ float lrcore(float c, float raw, float eps) {
   return c;
 }
 
+// LRcore lines that merge and split through LDS (up to 16 elements per thread
+// without a register-resident plan, and 2048 points) take their rows through
+// buffers: fewer registers (2048 points 125 -> 83, 810 points 78 -> 70), ms:
+// 1.104 -> 0.936 at 96 x 2048 x 2048, 0.161 -> 0.148 at 128 x 512 x 810,
+// 0.126 -> 0.118 for 48 stacks of 64 x 128 x 128.  Lines split by shuffles keep
+// addresses: 512 and 1024 points measured the same both ways (0.083; 0.593
+// against 0.597), 384 and 768 slower (0.142 -> 0.149, 0.124 -> 0.132), and the
+// R2C and update passes slower by 2% at 1024 points.
+constexpr bool lr_buf(int N) { return !x_shape(N, -1, XK_LR).SHUFFLE; }
+
 template <int N>
 __global__ void __launch_bounds__((XCfg<N, XK_LR>::THREADS))
     k_x_lrcore(float2* __restrict__ S, const float* __restrict__ raw, long rows, long pitch,
@@ -475,23 +529,49 @@ __global__ void __launch_bounds__((XCfg<N, XK_LR>::THREADS))
   __shared__ float2 lds[C::NL * C::LS];
   const int tid = threadIdx.x;
   const int l = tid / C::TPT, p = tid % C::TPT;
-  const long r0 = 2 * ((long)blockIdx.x * C::NL + l);
-  const bool v0 = r0 < rows, v1 = r0 + 1 < rows;
   float2* line = lds + l * C::LS;
   float2 v[C::E];
-  merge_load<N, XK_LR>(v, line, p, S, r0, pitch, v0, v1);
-  fft_line<N, C::TPT, 1, true>(v, line, p, tw);
+  const long rb = 2 * (long)blockIdx.x * C::NL, r0 = rb + 2 * l;  // the workgroup's first row, this line's
+  if constexpr (lr_buf(N)) {
+    const int nr = rows - rb < 2 * C::NL ? (int)(rows - rb) : 2 * C::NL;
+    const int pitch8 = (int)pitch * 8;
+    const RowsBuf<C::TPT> spec{SlabBuf(S + rb * pitch, nr * pitch8), 2 * l * pitch8 + 8 * p, pitch8};
+    merge_load<N, XK_LR>(v, line, p, spec);
+    fft_line<N, C::TPT, 1, true>(v, line, p, tw);
+    // the stack's loads stay behind the transform: otherwise they are issued
+    // before its last stage and held in registers (2048 points: 159, and
+    // 1.559 ms at 96 x 2048 x 2048)
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    const SlabBuf rw(raw + rb * N, nr * N * 4);
+    const int ro = (2 * l * N + p) * 4;
 #pragma unroll
-  for (int m = 0; m < C::E; ++m) {
-    const int i = p + m * C::TPT;
-    const float ra = v0 ? ld_stream<NTX>(raw + r0 * N + i) : 0.f;
-    const float rb = v1 ? ld_stream<NTX>(raw + (r0 + 1) * N + i) : 0.f;
-    v[m] = make_float2(lrcore(v[m].x, ra, eps), lrcore(v[m].y, rb, eps));
+    for (int m = 0; m < C::E; ++m) {
+      const float ra = rw.template load1<NTX>(ro, m * C::TPT * 4);
+      const float rc = rw.template load1<NTX>(ro, (m * C::TPT + N) * 4);
+      v[m] = make_float2(lrcore(v[m].x, ra, eps), lrcore(v[m].y, rc, eps));
+    }
+    __syncthreads();
+    fft_line<N, C::TPT, 1, false>(v, line, p, tw);
+    __syncthreads();
+    split_store<N, XK_LR>(v, line, p, spec);
+  } else {
+    const bool v0 = r0 < rows, v1 = r0 + 1 < rows;
+    const RowsPtr<C::TPT> spec{S + r0 * pitch + p, pitch, v0, v1};
+    merge_load<N, XK_LR>(v, line, p, spec);
+    fft_line<N, C::TPT, 1, true>(v, line, p, tw);
+#pragma unroll
+    for (int m = 0; m < C::E; ++m) {
+      const int i = p + m * C::TPT;
+      const float ra = v0 ? ld_stream<NTX>(raw + r0 * N + i) : 0.f;
+      const float rc = v1 ? ld_stream<NTX>(raw + (r0 + 1) * N + i) : 0.f;
+      v[m] = make_float2(lrcore(v[m].x, ra, eps), lrcore(v[m].y, rc, eps));
+    }
+    __syncthreads();
+    fft_line<N, C::TPT, 1, false>(v, line, p, tw);
+    __syncthreads();
+    split_store<N, XK_LR>(v, line, p, spec);
   }
-  __syncthreads();
-  fft_line<N, C::TPT, 1, false>(v, line, p, tw);
-  __syncthreads();
-  split_store<N, XK_LR>(v, line, p, S, r0, pitch, v0, v1);
 }
 
 // Deterministic workgroup sum of two doubles; out[0], out[1] written by
@@ -570,7 +650,7 @@ __global__ void __launch_bounds__(XCfg<N>::THREADS)
   const bool v0 = r0 < rows, v1 = r0 + 1 < rows;
   float2* line = lds + l * C::LS;
   float2 v[C::E];
-  merge_load<N>(v, line, p, S, r0, pitch, v0, v1);
+  merge_load<N>(v, line, p, RowsPtr<C::TPT>{const_cast<float2*>(S) + r0 * pitch + p, pitch, v0, v1});
   fft_line<N, C::TPT, 1, true>(v, line, p, tw);
   // all loads are issued before any store (G is read, then overwritten)
   float ya[C::E], yb[C::E], ga[C::E], gb[C::E];
@@ -662,32 +742,6 @@ __device__ __forceinline__ int support_ky(const OtfSupport& s, long c) {
   const float d = s.r2 - kx * kx;
   return d >= 0.f ? (int)(sqrtf(d) * s.iky) + 1 : -1;
 }
-
-// One slab of a spectrum as a buffer resource (32-bit byte offsets, scalar
-// row offsets): a thread keeps one offset for all its loads and stores
-// instead of a 64-bit address each, and a load at kNoRow returns zero without
-// touching memory, so skipping rows needs no branches.  The inverse y pass
-// with a branch per skipped row needs 75 registers at 1024 points, which
-// leaves one workgroup per CU instead of two (0.393 ms, every row read 0.382,
-// this form 0.357).  Registers of the y transforms: 64 to 2048 points 60-92
-// -> 56-81, of the z filters 92-142 -> 84-126 at 64 to 192 points.
-constexpr int kNoRow = -1;  // outside every slab
-typedef unsigned u2v __attribute__((ext_vector_type(2)));
-struct SlabBuf {
-  __amdgpu_buffer_rsrc_t rs;
-  __device__ __forceinline__ SlabBuf(float2* slab, int bytes)
-      : rs(__builtin_amdgcn_make_buffer_rsrc(slab, 0, bytes, 0x00020000)) {}
-  template <bool NT> __device__ __forceinline__ float2 load(int off, int row_off) const {
-    const u2v t = __builtin_amdgcn_raw_buffer_load_b64(rs, off, row_off, NT ? 2 : 0);
-    return make_float2(__uint_as_float(t.x), __uint_as_float(t.y));
-  }
-  template <bool NT> __device__ __forceinline__ void store(int off, int row_off, float2 v) const {
-    u2v t;
-    t.x = __float_as_uint(v.x);
-    t.y = __float_as_uint(v.y);
-    __builtin_amdgcn_raw_buffer_store_b64(t, rs, off, row_off, NT ? 2 : 0);
-  }
-};
 
 // The 256-point forward transform keeps plain addresses: with buffers the
 // compiler fuses the other product of two terms of its radix-16 stages into

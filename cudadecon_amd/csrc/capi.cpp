@@ -1128,7 +1128,8 @@ int cudaDecon_batch_get(cudaDecon_batch* h, int i, float* X) {
   return guard([&]() -> int {
     if (!h || !X || i < 0 || i >= (int)h->b.engines.size()) fail("cudaDecon_batch_get: bad argument");
     RLEngine& e = *h->b.engines[i];
-    CDN_HIP(hipMemcpy(X, e.result(), sizeof(float) * e.fft.nvox, hipMemcpyDeviceToHost));
+    // every run has ended (Batch::run waits for it)
+    copy_to_host(h->b.streams.back(), X, e.result(), sizeof(float) * e.fft.nvox);
     return 1;
   });
 }

@@ -11,7 +11,7 @@
 
 namespace cdn {
 
-// memcpy split over host threads (slices of at least 2 MB, at most 8
+// memcpy split over host threads (slices of at least 512 KB, at most 8
 // threads, the caller's included).  The workers start with the pool and wait
 // for the next job until it is destroyed.  Starting threads for every 32 MB
 // chunk instead halved the rate of a chunked memcpy on an 8-core host (22
@@ -42,9 +42,10 @@ class CopyPool {
   }
   CopyPool(const CopyPool&) = delete;
   CopyPool& operator=(const CopyPool&) = delete;
+  static constexpr size_t kSlice = 512UL << 10;
   size_t threads() const { return th_.size() + 1; }
   void copy(void* dst, const void* src, size_t n) {
-    const size_t nt = std::min<size_t>(th_.size() + 1, std::max<size_t>(1, n / (2UL << 20)));
+    const size_t nt = std::min<size_t>(th_.size() + 1, std::max<size_t>(1, n / kSlice));
     if (nt <= 1) {
       std::memcpy(dst, src, n);
       return;

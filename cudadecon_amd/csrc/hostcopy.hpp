@@ -2,9 +2,9 @@
 //
 // Measured on an MI355X host for 1 GiB: pageable hipMemcpy 26 GB/s to the
 // device and 17 GB/s back, pinned 57 GB/s both ways, one host thread's
-// memcpy 29 GB/s.  Large copies therefore go through two pinned staging
-// buffers: the DMA of one chunk overlaps several host threads copying the
-// other chunk between the caller's memory and the pinned buffer.
+// memcpy 29 GB/s.  Copies of some size therefore go through pinned staging
+// buffers: the DMA of one chunk overlaps several host threads copying another
+// chunk between the caller's memory and its pinned buffer.
 #pragma once
 
 #include <hip/hip_runtime.h>

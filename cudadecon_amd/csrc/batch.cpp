@@ -33,6 +33,7 @@
 
 #include <algorithm>
 #include <cfloat>
+#include <limits>
 #include <map>
 
 namespace cdn {
@@ -182,24 +183,38 @@ void Batch::build_groups() {
     std::map<ZKey, const float2*> ztw;
     std::map<int, long> ytot;
     std::map<ZKey, long> ztot;
+    // tile width of a group: by its largest column count
+    std::map<int, long> ycols;
+    std::map<ZKey, long> zcols;
     std::map<ZKey, bool> zbuf;
+    for (int p = P1.p0; p < P1.p1; ++p) {
+      const RLEngine& e = *engines[order[p]];
+      const ZKey key{e.fft.nz, e.otf.ra != 0};
+      long& yc = ycols[e.fft.ny];
+      yc = std::max(yc, (long)e.fft.nxh);
+      const bool buf = z_ragged_buf(e.fft.nz, (long)e.fft.ny * e.fft.pitch);
+      zbuf[key] = (zcols[key] == 0 || zbuf[key]) && buf;
+      zcols[key] = std::max(zcols[key], (long)e.fft.nxh);
+    }
+    for (auto& kv : ycols) kv.second = y_tile_cols(kv.first, kv.second);
+    for (auto& kv : zcols)
+      kv.second = z_tile_cols(kv.first.first, zbuf[kv.first] ? kv.second : std::numeric_limits<long>::max());
     for (int p = P1.p0; p < P1.p1; ++p) {
       const int i = order[p];
       const RLEngine& e = *engines[i];
       const Fft3& F = e.fft;
       float2* S = a_spec.as<float2>() + soff[i];
       {
-        const long L = col_tile_cols(F.ny), nt = (F.nxh + L - 1) / L;
+        const long L = ycols[F.ny], nt = (F.nxh + L - 1) / L;
         ColSeg sg{S, F.nxh, F.pitch, (long)F.ny * F.pitch, nt, ytot[F.ny], e.otf.params(e.table, 1.0).sup};
         ys[F.ny].push_back(sg);
         ytot[F.ny] += (long)F.nz * nt;
         ytw[F.ny] = F.twy.as<float2>();
       }
       {
-        const long L = col_tile_cols(F.nz), nt = (F.nxh + L - 1) / L;
         const OtfParams op = e.otf.params(e.table, 1.0 / (double)F.nvox);
         const ZKey key{F.nz, op.ra != 0};
-        zbuf[key] = (ztot[key] == 0 || zbuf[key]) && z_ragged_buf(F.nz, (long)F.ny * F.pitch);
+        const long L = zcols[key], nt = (F.nxh + L - 1) / L;
         ZSeg sg{S, F.nxh, (long)F.ny * F.pitch, F.pitch, nt, F.ny, ztot[key], op};
         zs[key].push_back(sg);
         ztot[key] += (long)F.ny * nt;
@@ -211,6 +226,7 @@ void Batch::build_groups() {
       g.len = kv.first;
       g.nseg = (int)kv.second.size();
       g.total = ytot[kv.first];
+      g.cols = ycols[kv.first];
       g.tw = ytw[kv.first];
       g.segs.ensure(sizeof(ColSeg) * kv.second.size());
       CDN_HIP(hipMemcpy(g.segs.p, kv.second.data(), sizeof(ColSeg) * kv.second.size(), hipMemcpyHostToDevice));
@@ -224,6 +240,7 @@ void Batch::build_groups() {
       g.buf = zbuf[kv.first];
       g.nseg = (int)kv.second.size();
       g.total = ztot[kv.first];
+      g.cols = zcols[kv.first];
       g.tw = ztw[kv.first];
       g.segs.ensure(sizeof(ZSeg) * kv.second.size());
       CDN_HIP(hipMemcpy(g.segs.p, kv.second.data(), sizeof(ZSeg) * kv.second.size(), hipMemcpyHostToDevice));
@@ -293,14 +310,14 @@ void Batch::enqueue_partition(const Partition& P, hipStream_t st, int iters, hip
     CDN_HIP(hipEventRecord(mark, st));
     for (int f = 0; f < 2; ++f) {
       for (const ColGroup& g : P.yg)
-        launch_col_ragged(g.len, 0, st, g.segs.as<ColSeg>(), g.nseg, g.total, g.tw, grid_cap);
+        launch_col_ragged(g.len, 0, st, g.segs.as<ColSeg>(), g.nseg, g.total, g.cols, g.tw, grid_cap);
       CDN_HIP(hipEventRecord(mark, st));
       for (const ColGroup& g : P.zg)
-        launch_z_ragged(g.len, st, g.segs.as<ZSeg>(), g.nseg, g.total, f, g.tw, grid_cap, g.ra,
+        launch_z_ragged(g.len, st, g.segs.as<ZSeg>(), g.nseg, g.total, g.cols, f, g.tw, grid_cap, g.ra,
                         g.buf);
       CDN_HIP(hipEventRecord(mark, st));
       for (const ColGroup& g : P.yg)
-        launch_col_ragged(g.len, 1, st, g.segs.as<ColSeg>(), g.nseg, g.total, g.tw, grid_cap);
+        launch_col_ragged(g.len, 1, st, g.segs.as<ColSeg>(), g.nseg, g.total, g.cols, g.tw, grid_cap);
       CDN_HIP(hipEventRecord(mark, st));
       if (f == 0) {
         for (const XGroup& g : P.xg)

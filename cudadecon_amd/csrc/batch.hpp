@@ -60,6 +60,7 @@ struct Batch {
     bool ra = false;  // z groups: every table rotationally averaged
     bool buf = true;  // z groups: launch_z_ragged's buf
     long total = 0;
+    long cols = 0;  // columns per tile
     const float2* tw = nullptr;
     DevBuf segs;
   };

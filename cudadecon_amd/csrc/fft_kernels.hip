@@ -250,35 +250,79 @@ bool fft_balanced_cols(int len, long ncols, FftVariant* v) {
   return true;
 }
 
-// tuned variant of the length, else one tile of all columns, else built in
-static bool col_variant(int len, long ncols, FftVariant* v) {
-  if (fft_get_variant(len, v)) return true;
-  return fft_balanced_cols(len, ncols, v);
+// Tiles of 16 columns (128-byte rows) instead of 32 or 64, built for lengths
+// 64, 128 and 256.  Up to 160 columns they leave less of the last tile empty
+// (65 columns: 80 instead of 96 or 128), cut the support's edge finer and give
+// more, smaller workgroups; with more columns the y passes of 64 and 256 still
+// gain, while the z filters lose the longer rows of their far-apart planes.
+// ms per launch, wide -> 16: z filter of 64, 65 columns (48 stacks of
+// 64 x 128 x 128) 0.107 -> 0.095, 129 columns 0.0157 -> 0.0151, 513 columns
+// 0.102 -> 0.106; of 128, 129 columns 0.0212 -> 0.0196, 257 columns 0.0502 ->
+// 0.0518; of 256, 129 columns 0.0355 -> 0.0334, 513 columns 0.354 -> 0.384;
+// y of 256, 1025 columns 0.072 -> 0.066, 129 columns 0.0136 -> 0.0119; y of
+// 128, 65 columns 0.077 -> 0.074, 513 columns 0.0442 -> 0.0450; y of 64 0.0259
+// -> 0.0253 at 513 columns.  Lengths 96 and 192 (24 elements per thread, 64
+// threads in such a tile): z 0.0166 -> 0.0173.
+constexpr int kNarrowCols = 16;
+constexpr long kNarrowMax = 160;
+#define CDN_NARROW_LENGTHS(X) X(64) X(128) X(256)
+static bool y_narrow(int len, long ncols) {
+  return len == 64 || len == 256 || (len == 128 && ncols <= kNarrowMax);
+}
+static bool z_narrow(int len, long ncols) {
+  return (len == 64 || len == 128 || len == 256) && ncols <= kNarrowMax;
 }
 
-void fft_prepare_cols(int len, long ncols) {
+// How a column pass runs: the tuned variant of the length, else narrow tiles,
+// else one tile of all columns, else the length's own shape.
+struct ColRun {
+  CShape cs;
+  bool jit, narrow;
   FftVariant v;
-  if (fft_get_variant(len, &v) || !fft_balanced_cols(len, ncols, &v)) return;
+};
+static ColRun col_run(int len, long ncols, bool narrow) {
+  ColRun r{};
+  r.jit = fft_get_variant(len, &r.v);
+  r.narrow = !r.jit && narrow;
+  if (!r.jit && !r.narrow) r.jit = fft_balanced_cols(len, ncols, &r.v);
+  r.cs = r.narrow ? c_shape(len, kNarrowCols) : c_shape(len, r.jit ? r.v.cols : -1, r.jit ? r.v.col_tpt : -1);
+  return r;
+}
+
+void fft_prepare_cols(int len, long ncols, bool z) {
+  FftVariant v;
+  if (fft_get_variant(len, &v) || (z ? z_narrow(len, ncols) : y_narrow(len, ncols))) return;
+  if (!fft_balanced_cols(len, ncols, &v)) return;
   // compile and load (grid 0: no launch) before any stream capture
   for (JitKernel k : {JK_COL_F, JK_COL_I, JK_Z_FILTER, JK_Z_FILTER_RA}) jit_launch(len, k, 0, 1, nullptr, nullptr, v);
 }
 
 void launch_col_fft(int len, int inverse, hipStream_t st, float2* S, long ncols, long line_stride,
                     long outer_stride, long n_outer, const float2* tw, const OtfSupport& sup) {
-  FftVariant tv;
-  const bool tuned = col_variant(len, ncols, &tv);
-  const CShape cs = c_shape(len, tuned ? tv.cols : -1, tuned ? tv.col_tpt : -1);
-  long ntiles = (ncols + cs.L - 1) / cs.L;
-  const unsigned grid = grid1(ntiles * n_outer);
-  OtfSupport sp = sup;
   // a slab's rows by 32-bit offsets (always the case for y transforms: at
   // most 16384 rows of 8208 columns)
   const bool buf = (double)len * (double)line_stride * 8.0 < 2147483648.0;
+  const ColRun run = col_run(len, ncols, buf && y_narrow(len, ncols));
+  const CShape cs = run.cs;
+  long ntiles = (ncols + cs.L - 1) / cs.L;
+  const unsigned grid = grid1(ntiles * n_outer);
+  OtfSupport sp = sup;
   if (!buf && sp.r2 >= 0.f) fail("launch_col_fft: support bound on a slab of 2 GiB or more");
   void* args[] = {&S, &ncols, &line_stride, &outer_stride, &ntiles, &sp, &tw};
   const JitKernel jk = inverse ? (buf ? JK_COL_I : JK_COL_IW) : (buf ? JK_COL_F : JK_COL_FW);
-  if (tuned) {
-    jit_launch(len, jk, grid, cs.THREADS, st, args, tv);
+  if (run.jit) {
+    jit_launch(len, jk, grid, cs.THREADS, st, args, run.v);
+  } else if (run.narrow) {
+    switch (len) {
+#define CDN_CASE(N)                                                                                                  \
+  case N: {                                                                                                          \
+    auto* k = inverse ? k_col<N, true, true, kNarrowCols> : k_col<N, false, true, kNarrowCols>;                      \
+    hipLaunchKernelGGL(k, dim3(grid), dim3(cs.THREADS), 0, st, S, ncols, line_stride, outer_stride, ntiles, sp, tw); \
+    break;                                                                                                           \
+  }
+      CDN_NARROW_LENGTHS(CDN_CASE)
+#undef CDN_CASE
+    }
   } else {
     switch (len) {
 #define CDN_CASE(N)                                                                                                  \
@@ -305,9 +349,8 @@ bool z_ragged_buf(int nz, long line_stride) { return z_buf(c_shape(nz), line_str
 
 void launch_z_filter(int nz, hipStream_t st, float2* S, long ncols, long line_stride, long outer_stride, long ny,
                      int conj, const OtfParams& otf, const float2* tw, int nstacks, long stack_stride) {
-  FftVariant tv;
-  const bool tuned = col_variant(nz, ncols, &tv);
-  const CShape cs = c_shape(nz, tuned ? tv.cols : -1, tuned ? tv.col_tpt : -1);
+  const ColRun run = col_run(nz, ncols, z_narrow(nz, ncols) && z_buf(c_shape(nz), line_stride));
+  const CShape cs = run.cs;
   long ntiles = (ncols + cs.L - 1) / cs.L;
   if (nstacks < 1) fail("launch_z_filter: no stacks");
   const unsigned grid = grid1(ntiles * ny * nstacks);
@@ -316,8 +359,20 @@ void launch_z_filter(int nz, hipStream_t st, float2* S, long ncols, long line_st
   // the averaged-table kind for a rotationally averaged OTF
   const bool ra = op.ra != 0, buf = z_buf(cs, line_stride);
   const JitKernel jk = ra ? (buf ? JK_Z_FILTER_RA : JK_Z_FILTER_RA_W) : (buf ? JK_Z_FILTER : JK_Z_FILTER_W);
-  if (tuned) {
-    jit_launch(nz, jk, grid, cs.THREADS, st, args, tv);
+  if (run.jit) {
+    jit_launch(nz, jk, grid, cs.THREADS, st, args, run.v);
+  } else if (run.narrow) {
+    switch (nz) {
+#define CDN_CASE(N)                                                                                             \
+  case N: {                                                                                                     \
+    auto* k = ra ? k_z_filter<N, ZF_RA, true, kNarrowCols> : k_z_filter<N, ZF_ANY, true, kNarrowCols>;          \
+    hipLaunchKernelGGL(k, dim3(grid), dim3(cs.THREADS), 0, st, S, ncols, line_stride, outer_stride, ntiles, ny, \
+                       stack_stride, conj, op, tw);                                                             \
+    break;                                                                                                      \
+  }
+      CDN_NARROW_LENGTHS(CDN_CASE)
+#undef CDN_CASE
+    }
   } else {
     switch (nz) {
 #define CDN_CASE(N)                                                                                             \
@@ -337,7 +392,8 @@ void launch_z_filter(int nz, hipStream_t st, float2* S, long ncols, long line_st
   CDN_HIP(hipGetLastError());
 }
 
-long col_tile_cols(int len) { return c_shape(len).L; }
+long y_tile_cols(int len, long ncols) { return y_narrow(len, ncols) ? kNarrowCols : c_shape(len).L; }
+long z_tile_cols(int len, long ncols) { return z_narrow(len, ncols) ? kNarrowCols : c_shape(len).L; }
 
 void fft_prepare_ragged(int len) {
   if (fft_length_precompiled(len)) return;
@@ -355,70 +411,86 @@ static unsigned ragged_grid(long total, long cap) {
 }
 
 // the kernel instance for (inverse, persistent)
-template <int N>
-static void col_ragged_n(bool inv, bool pers, unsigned grid, unsigned threads, hipStream_t st, const ColSeg* segs,
-                         int nseg, long total, const float2* tw) {
-  if (inv && pers)
-    hipLaunchKernelGGL((k_col_ragged<N, true, true>), dim3(grid), dim3(threads), 0, st, segs, nseg, total, tw);
-  else if (inv)
-    hipLaunchKernelGGL((k_col_ragged<N, true, false>), dim3(grid), dim3(threads), 0, st, segs, nseg, total, tw);
-  else if (pers)
-    hipLaunchKernelGGL((k_col_ragged<N, false, true>), dim3(grid), dim3(threads), 0, st, segs, nseg, total, tw);
-  else
-    hipLaunchKernelGGL((k_col_ragged<N, false, false>), dim3(grid), dim3(threads), 0, st, segs, nseg, total, tw);
+template <int N, int COLS>
+static auto col_ragged_n(bool inv, bool pers) {
+  return inv ? (pers ? k_col_ragged<N, true, true, COLS> : k_col_ragged<N, true, false, COLS>)
+             : (pers ? k_col_ragged<N, false, true, COLS> : k_col_ragged<N, false, false, COLS>);
 }
 
-void launch_col_ragged(int len, int inverse, hipStream_t st, const ColSeg* segs, int nseg, long total,
+void launch_col_ragged(int len, int inverse, hipStream_t st, const ColSeg* segs, int nseg, long total, long cols,
                        const float2* tw, long grid_cap) {
   if (total <= 0) return;
-  const CShape cs = c_shape(len);
+  const bool narrow = cols != c_shape(len).L;
+  const CShape cs = c_shape(len, narrow ? (int)cols : -1);
   const unsigned grid = ragged_grid(total, grid_cap);
-  const bool pers = grid < total;
+  const bool inv = inverse != 0, pers = grid < total;
   void* args[] = {&segs, &nseg, &total, &tw};
-  switch (len) {
-#define CDN_CASE(N)                                                                      \
-  case N:                                                                                \
-    col_ragged_n<N>(inverse != 0, pers, grid, cs.THREADS, st, segs, nseg, total, tw); \
-    break;
-    CDN_FFT_LENGTHS(CDN_CASE)
+  void (*k)(const ColSeg*, int, long, const float2*) = nullptr;
+  if (narrow) {
+    switch (len) {
+#define CDN_CASE(N) \
+  case N: k = col_ragged_n<N, kNarrowCols>(inv, pers); break;
+      CDN_NARROW_LENGTHS(CDN_CASE)
 #undef CDN_CASE
-    default:
-      jit_launch(len, pers ? (inverse ? JK_COL_RAGGED_IP : JK_COL_RAGGED_FP) : (inverse ? JK_COL_RAGGED_I : JK_COL_RAGGED_F),
-                 grid, cs.THREADS, st, args);
+    }
+    if (!k || cols != kNarrowCols) fail("launch_col_ragged: no tile of " + std::to_string(cols) + " columns");
+  } else {
+    switch (len) {
+#define CDN_CASE(N) \
+  case N: k = col_ragged_n<N, 0>(inv, pers); break;
+      CDN_FFT_LENGTHS(CDN_CASE)
+#undef CDN_CASE
+    }
   }
+  if (k)
+    hipLaunchKernelGGL(k, dim3(grid), dim3(cs.THREADS), 0, st, segs, nseg, total, tw);
+  else
+    jit_launch(len, pers ? (inv ? JK_COL_RAGGED_IP : JK_COL_RAGGED_FP) : (inv ? JK_COL_RAGGED_I : JK_COL_RAGGED_F),
+               grid, cs.THREADS, st, args);
   CDN_HIP(hipGetLastError());
 }
 
 // the kernel instance for (persistent, kind, buffer addressing); stacks that
 // need 64-bit addresses fill the GPU one item per workgroup
-template <int N>
+template <int N, int COLS>
 static auto z_ragged_n(bool pers, bool ra, bool buf) {
-  if (!buf) return ra ? k_z_ragged<N, false, ZF_RA, false> : k_z_ragged<N, false, ZF_ANY, false>;
-  return pers ? (ra ? k_z_ragged<N, true, ZF_RA> : k_z_ragged<N, true, ZF_ANY>)
-              : (ra ? k_z_ragged<N, false, ZF_RA> : k_z_ragged<N, false, ZF_ANY>);
+  if (COLS == 0 && !buf) return ra ? k_z_ragged<N, false, ZF_RA, false> : k_z_ragged<N, false, ZF_ANY, false>;
+  return pers ? (ra ? k_z_ragged<N, true, ZF_RA, true, COLS> : k_z_ragged<N, true, ZF_ANY, true, COLS>)
+              : (ra ? k_z_ragged<N, false, ZF_RA, true, COLS> : k_z_ragged<N, false, ZF_ANY, true, COLS>);
 }
 
-void launch_z_ragged(int nz, hipStream_t st, const ZSeg* segs, int nseg, long total, int conj, const float2* tw,
-                     long grid_cap, bool ra, bool buf) {
+void launch_z_ragged(int nz, hipStream_t st, const ZSeg* segs, int nseg, long total, long cols, int conj,
+                     const float2* tw, long grid_cap, bool ra, bool buf) {
   if (total <= 0) return;
-  const CShape cs = c_shape(nz);
+  const bool narrow = cols != c_shape(nz).L;
+  const CShape cs = c_shape(nz, narrow ? (int)cols : -1);
   const unsigned grid = ragged_grid(total, buf ? grid_cap : 0);
   const bool pers = grid < total;
   void* args[] = {&segs, &nseg, &total, &conj, &tw};
-  switch (nz) {
-#define CDN_CASE(N)                                                                                        \
-  case N: {                                                                                                \
-    auto* k = z_ragged_n<N>(pers, ra, buf);                                                                \
-    hipLaunchKernelGGL(k, dim3(grid), dim3(cs.THREADS), 0, st, segs, nseg, total, conj, tw);               \
-    break;                                                                                                 \
-  }
-    CDN_FFT_LENGTHS(CDN_CASE)
+  void (*k)(const ZSeg*, int, long, int, const float2*) = nullptr;
+  if (narrow) {
+    switch (nz) {
+#define CDN_CASE(N) \
+  case N: k = z_ragged_n<N, kNarrowCols>(pers, ra, true); break;
+      CDN_NARROW_LENGTHS(CDN_CASE)
 #undef CDN_CASE
-    default: {
-      const JitKernel b[4] = {JK_Z_RAGGED, JK_Z_RAGGED_P, JK_Z_RAGGED_RA, JK_Z_RAGGED_P_RA};
-      const JitKernel w[2] = {JK_Z_RAGGED_W, JK_Z_RAGGED_RA_W};
-      jit_launch(nz, buf ? b[2 * ra + pers] : w[ra], grid, cs.THREADS, st, args);
     }
+    if (!k || !buf || cols != kNarrowCols)
+      fail("launch_z_ragged: no tile of " + std::to_string(cols) + " columns");
+  } else {
+    switch (nz) {
+#define CDN_CASE(N) \
+  case N: k = z_ragged_n<N, 0>(pers, ra, buf); break;
+      CDN_FFT_LENGTHS(CDN_CASE)
+#undef CDN_CASE
+    }
+  }
+  if (k) {
+    hipLaunchKernelGGL(k, dim3(grid), dim3(cs.THREADS), 0, st, segs, nseg, total, conj, tw);
+  } else {
+    const JitKernel b[4] = {JK_Z_RAGGED, JK_Z_RAGGED_P, JK_Z_RAGGED_RA, JK_Z_RAGGED_P_RA};
+    const JitKernel w[2] = {JK_Z_RAGGED_W, JK_Z_RAGGED_RA_W};
+    jit_launch(nz, buf ? b[2 * ra + pers] : w[ra], grid, cs.THREADS, st, args);
   }
   CDN_HIP(hipGetLastError());
 }

@@ -57,8 +57,9 @@ void fft_set_variant(int n, const FftVariant& v);
 // fits (v: the variant); the column launchers use it unless the length has
 // a tuned variant.
 bool fft_balanced_cols(int len, long ncols, FftVariant* v);
-// compile and load the kernels those launches will need (no GPU work)
-void fft_prepare_cols(int len, long ncols);
+// compile and load the kernels those launches will need (no GPU work); z: as
+// a z filter, else as a y transform
+void fft_prepare_cols(int len, long ncols, bool z);
 bool fft_get_variant(int n, FftVariant* v);
 // While one exists on this thread, every launch uses the built-in kernels of
 // its length: no tuned or single-tile variant, whose run-time compiled code
@@ -86,18 +87,19 @@ void launch_z_filter(int nz, hipStream_t st, float2* S, long ncols, long line_st
 
 // Column passes spanning stacks of different shapes: one launch for every
 // stack whose transform length is `len`, segs (device) one per stack with
-// items numbered by tiles of col_tile_cols(len) columns, `total` items in
-// all.  grid_cap > 0 bounds the workgroups, which then walk the items.
-long col_tile_cols(int len);
+// items numbered by tiles of `cols` columns (y_tile_cols / z_tile_cols of the
+// launch's largest column count), `total` items in all.  grid_cap > 0 bounds the workgroups, which then walk the items.
+long y_tile_cols(int len, long ncols);
+long z_tile_cols(int len, long ncols);
 // compile and load the run-time kernels the ragged launches of a length not
 // built in will use (no GPU work; call before any stream capture)
 void fft_prepare_ragged(int len);
 void launch_col_ragged(int len, int inverse, hipStream_t st, const ColSeg* segs, int nseg, long total,
-                       const float2* tw, long grid_cap = 0);
+                       long cols, const float2* tw, long grid_cap = 0);
 // ra: every segment's OTF is rotationally averaged (the kernel kind the
 // one-stack z filter uses for such a table)
-void launch_z_ragged(int nz, hipStream_t st, const ZSeg* segs, int nseg, long total, int conj, const float2* tw,
-                     long grid_cap = 0, bool ra = false, bool buf = true);
+void launch_z_ragged(int nz, hipStream_t st, const ZSeg* segs, int nseg, long total, long cols, int conj,
+                     const float2* tw, long grid_cap = 0, bool ra = false, bool buf = true);
 // whether a stack's z filter can address its planes (line_stride apart) by
 // 32-bit offsets: buf above, for every segment of the launch
 bool z_ragged_buf(int nz, long line_stride);

@@ -242,8 +242,9 @@ template <int N, int K = XK_PLAIN> struct XCfg {
 #ifndef CDN_SPLIT_LDS
 #define CDN_SPLIT_LDS 1
 #endif
-template <int N> struct CCfg {
-  static constexpr CShape S = c_shape(N);
+// COLS > 0: that many columns per tile instead of the length's own width.
+template <int N, int COLS = 0> struct CCfg {
+  static constexpr CShape S = c_shape(N, COLS > 0 ? COLS : -1);
   static constexpr int TPT = S.TPT, L = S.L, THREADS = S.THREADS, E = S.E;
   static constexpr bool HALF = CDN_SPLIT_LDS != 0 && plan_exact(N, S.TPT);
   static constexpr int LDS = HALF ? (N * L + 1) / 2 : N * L;  // float2 elements
@@ -713,10 +714,10 @@ __device__ __forceinline__ long xcd_logical_block(long b, long G) {
 // y / z column passes: thread (l, p) holds column l's elements p + m TPT
 // ---------------------------------------------------------------------------
 // the transform of column l of a tile (LDS as declared by the kernel)
-template <int N, bool INV>
-__device__ __forceinline__ void col_line(float2 (&v)[CCfg<N>::E], float2* lds, int l, int p,
+template <int N, bool INV, int COLS = 0>
+__device__ __forceinline__ void col_line(float2 (&v)[(CCfg<N, COLS>::E)], float2* lds, int l, int p,
                                          const float2* __restrict__ tw) {
-  using C = CCfg<N>;
+  using C = CCfg<N, COLS>;
   if constexpr (C::HALF) {
     fft_line_half<N, C::TPT, C::L, INV>(v, reinterpret_cast<float*>(lds) + l, p, tw);
   } else {
@@ -753,11 +754,11 @@ constexpr bool col_buf(int N, bool inv) { return N != 256 || inv; }
 // tile lb (slab-major) of a column pass; lds as declared by the kernel.  sup:
 // for the y transforms around a z filter, its OTF's support.  BUF: a
 // slab (N rows) spans less than 2^31 bytes.
-template <int N, bool INV, bool BUF>
+template <int N, bool INV, bool BUF, int COLS>
 __device__ __forceinline__ void col_tile(float2* lds, float2* __restrict__ S, long ncols, long line_stride,
                                          long outer_stride, long ntiles, long lb, const OtfSupport& sup,
                                          const float2* __restrict__ tw) {
-  using C = CCfg<N>;
+  using C = CCfg<N, COLS>;
   const int tid = threadIdx.x;
   const int l = tid % C::L, p = tid / C::L;
   const long outer = lb / ntiles, tile = lb - outer * ntiles;
@@ -774,7 +775,7 @@ __device__ __forceinline__ void col_tile(float2* lds, float2* __restrict__ S, lo
 #pragma unroll
     for (int m = 0; m < C::E; ++m)
       v[m] = slab.template load<NTCL>(INV ? live(p + m * C::TPT) : off, m * C::TPT * ls8);
-    col_line<N, INV>(v, lds, l, p, tw);
+    col_line<N, INV, COLS>(v, lds, l, p, tw);
 #pragma unroll
     for (int m = 0; m < C::E; ++m)
       slab.template store<NTCS>(INV ? off : live(p + m * C::TPT), m * C::TPT * ls8, v[m]);
@@ -783,7 +784,7 @@ __device__ __forceinline__ void col_tile(float2* lds, float2* __restrict__ S, lo
 #pragma unroll
     for (int m = 0; m < C::E; ++m)
       v[m] = valid ? ld_stream<NTCL>(base + (long)(p + m * C::TPT) * line_stride) : make_float2(0.f, 0.f);
-    col_line<N, INV>(v, lds, l, p, tw);
+    col_line<N, INV, COLS>(v, lds, l, p, tw);
     if (valid) {
 #pragma unroll
       for (int m = 0; m < C::E; ++m) st_stream<NTCS>(base + (long)(p + m * C::TPT) * line_stride, v[m]);
@@ -791,13 +792,14 @@ __device__ __forceinline__ void col_tile(float2* lds, float2* __restrict__ S, lo
   }
 }
 
-template <int N, bool INV, bool BUF = true>
-__global__ void __launch_bounds__(CCfg<N>::THREADS)
+template <int N, bool INV, bool BUF = true, int COLS = 0>
+__global__ void __launch_bounds__((CCfg<N, COLS>::THREADS))
     k_col(float2* __restrict__ S, long ncols, long line_stride, long outer_stride, long ntiles, OtfSupport sup,
           const float2* __restrict__ tw) {
-  __shared__ float2 lds[CCfg<N>::LDS];
-  col_tile<N, INV, BUF>(lds, S, ncols, line_stride, outer_stride, ntiles,
-                        xcd_logical_block<CCfg<N>::L>(blockIdx.x, gridDim.x), sup, tw);
+  using C = CCfg<N, COLS>;
+  __shared__ float2 lds[C::LDS];
+  col_tile<N, INV, BUF, COLS>(lds, S, ncols, line_stride, outer_stride, ntiles,
+                              xcd_logical_block<C::L>(blockIdx.x, gridDim.x), sup, tw);
 }
 
 // segment holding work item `it`: the last whose item0 <= it (segs[0].item0 = 0)
@@ -820,16 +822,16 @@ __device__ __forceinline__ int find_seg(const Seg* __restrict__ segs, int n, lon
 // 8 so an item runs on the XCD the block order assumes, workgroup b taking
 // items b, b + gridDim.x, ...  (The loop keeps more values live: 112 against
 // 61 VGPRs at length 1024, so it is an option, not the default.)
-template <int N, bool INV, bool PERSIST>
-__global__ void __launch_bounds__(CCfg<N>::THREADS)
+template <int N, bool INV, bool PERSIST, int COLS = 0>
+__global__ void __launch_bounds__((CCfg<N, COLS>::THREADS))
     k_col_ragged(const ColSeg* __restrict__ segs, int nseg, long total, const float2* __restrict__ tw) {
-  __shared__ float2 lds[CCfg<N>::LDS];
+  using C = CCfg<N, COLS>;
+  __shared__ float2 lds[C::LDS];
   long it = blockIdx.x;
   do {
-    const long lb = xcd_logical_block<CCfg<N>::L>(it, total);
+    const long lb = xcd_logical_block<C::L>(it, total);
     const ColSeg& g = segs[find_seg(segs, nseg, lb)];
-    col_tile<N, INV, true>(lds, g.S, g.ncols, g.line_stride, g.outer_stride, g.ntiles, lb - g.item0, g.sup,
-                     tw);
+    col_tile<N, INV, true, COLS>(lds, g.S, g.ncols, g.line_stride, g.outer_stride, g.ntiles, lb - g.item0, g.sup, tw);
     if constexpr (!PERSIST) break;
     __syncthreads();  // the next item's exchanges reuse lds
     it += gridDim.x;
@@ -851,9 +853,9 @@ enum ZfKind : int { ZF_ANY = 0, ZF_RA = 1 };
 #ifndef CDN_ZF_WAVES
 #define CDN_ZF_WAVES 0
 #endif
-constexpr int zf_waves(int N, int kind = ZF_ANY) {
+constexpr int zf_waves(int N, int kind = ZF_ANY, int cols = 0) {
   if (CDN_ZF_WAVES > 0) return CDN_ZF_WAVES;
-  const CShape c = c_shape(N);
+  const CShape c = c_shape(N, cols > 0 ? cols : -1);
   const bool half = CDN_SPLIT_LDS != 0 && plan_exact(N, c.TPT);
   if (N == 256 && c.THREADS == 512 && half && N * c.L * 4 <= 32768) return 6;
   if (N == 512 && kind == ZF_RA && c.THREADS == 512 && c.E == 16 && half) return 6;
@@ -891,14 +893,16 @@ template <int N, int KIND> struct ZRows {
 // filter_kernel / filterConj_kernel (src/RLgpuImpl.cu:331-350) with the OTF
 // value computed on the fly as in dev_otfinterpolate (src/RLgpuImpl.cu:228-329)
 // BUF: TPT rows (planes) span less than 2^31 bytes (z_buf).
-template <int N, int KIND = ZF_ANY, bool BUF = true>
-__global__ void __launch_bounds__(CCfg<N>::THREADS) __attribute__((amdgpu_waves_per_eu(zf_waves(N, KIND))))
+template <int N, int KIND = ZF_ANY, bool BUF = true, int COLS = 0>
+__global__ void __launch_bounds__((CCfg<N, COLS>::THREADS))
+    __attribute__((amdgpu_waves_per_eu(zf_waves(N, KIND, COLS))))
     k_z_filter(float2* __restrict__ S, long ncols, long line_stride, long outer_stride, long ntiles, long ny,
                long stack_stride, int conj, OtfParams otf, const float2* __restrict__ tw) {
-  using C = CCfg<N>;
+  using C = CCfg<N, COLS>;
   constexpr int RS = ZRows<N, KIND>::R;
   constexpr int PER = RS > 0 ? (RS * N + C::THREADS - 1) / C::THREADS : 1;
   constexpr bool ZRA = KIND == ZF_RA, ZBUF = BUF;
+  constexpr int ZCOLS = COLS;
   __shared__ float2 lds[C::LDS];
   __shared__ float2 otf_rows[RS > 0 ? RS * N : 1];
   const long lb = xcd_logical_block<C::L>(blockIdx.x, gridDim.x);
@@ -911,10 +915,11 @@ __global__ void __launch_bounds__(CCfg<N>::THREADS) __attribute__((amdgpu_waves_
 // and OTFs in one launch (ZSeg per stack); items and PERSIST as k_col_ragged.
 // KIND as k_z_filter's (ZF_RA: every segment's table is rotationally
 // averaged), so that each stack runs the code its one-stack engine runs.
-template <int N, bool PERSIST, int KIND = ZF_ANY, bool BUF = true>
-__global__ void __launch_bounds__(CCfg<N>::THREADS) __attribute__((amdgpu_waves_per_eu(zf_waves(N, KIND))))
+template <int N, bool PERSIST, int KIND = ZF_ANY, bool BUF = true, int COLS = 0>
+__global__ void __launch_bounds__((CCfg<N, COLS>::THREADS))
+    __attribute__((amdgpu_waves_per_eu(zf_waves(N, KIND, COLS))))
     k_z_ragged(const ZSeg* __restrict__ segs, int nseg, long total, int conj, const float2* __restrict__ tw) {
-  using C = CCfg<N>;
+  using C = CCfg<N, COLS>;
   constexpr int RS = ZRows<N, KIND>::R;
   constexpr int PER = RS > 0 ? (RS * N + C::THREADS - 1) / C::THREADS : 1;
   __shared__ float2 lds[C::LDS];
@@ -928,6 +933,7 @@ __global__ void __launch_bounds__(CCfg<N>::THREADS) __attribute__((amdgpu_waves_
     const long ntiles = g->ntiles, ny = g->ny, stack_stride = 0, lb = gi - g->item0;
     const OtfParams& otf = g->otf;
     constexpr bool ZRA = KIND == ZF_RA, ZBUF = BUF;
+    constexpr int ZCOLS = COLS;
     do {
 #include "zf_tile_body.inc"
     } while (false);

@@ -41,3 +41,20 @@ def test_filter_with_bounded_support_matches_oracle(cdn, orc, shape, scale, nr):
         ref = orc.filt(v.astype(np.float64), H, conj=conj)
         got = cdn.filter_volume(v, tab, ks, conj=conj)
         assert np.abs(got - ref).max() <= 1e-5 * np.abs(ref).max()
+
+
+# tiles of 16 columns (csrc/fft_kernels.hip, y_narrow and z_narrow): exactly one
+# tile, one column more, several with a remainder, the last count with narrow z
+# tiles and the first without
+@pytest.mark.parametrize("shape", [(64, 128, 30), (128, 64, 32), (256, 128, 64), (128, 256, 315), (64, 128, 320)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_narrow_tiles_match_oracle(cdn, orc, shape):
+    nz, ny, nx = shape
+    rng = np.random.default_rng(nx)
+    tab = (rng.uniform(0.2, 1.0, (9, 12)) + 1j * rng.uniform(-0.5, 0.5, (9, 12))).astype(np.complex64)
+    ks = tuple(np.float32(v) for v in (0.99913 * 16 / nx, 1.00071 * 16 / ny, 12.0 / nz))
+    v = rng.uniform(0, 100, shape).astype(np.float32)
+    print("narrow", shape, flush=True)
+    ref = orc.filt(v.astype(np.float64), orc.otf_interp(tab, (9, 1, 12), (nx, ny, nz), ks))
+    got = cdn.filter_volume(v, tab, ks)
+    assert np.abs(got - ref).max() <= 1e-5 * np.abs(ref).max()

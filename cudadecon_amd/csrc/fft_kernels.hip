@@ -263,10 +263,19 @@ bool fft_balanced_cols(int len, long ncols, FftVariant* v) {
 // 128, 65 columns 0.077 -> 0.074, 513 columns 0.0442 -> 0.0450; y of 64 0.0259
 // -> 0.0253 at 513 columns.  Lengths 96 and 192 (24 elements per thread, 64
 // threads in such a tile): z 0.0166 -> 0.0173.
+//
+// 2048-point y columns run 8 to a tile (64-byte rows); 16 of them with 64
+// threads and 32 elements each (one workgroup per CU) read whole 128-byte
+// lines: 0.693 -> 0.632 ms at 96 x 2048 x 2048, 0.180 -> 0.177 at
+// 64 x 2048 x 768 (1600 workgroups), but 0.0425 -> 0.0477 at 32 x 2048 x 256 (288
+// workgroups, a second round of 32), so from 4 rounds of 256 workgroups on.
 constexpr int kNarrowCols = 16;
 constexpr long kNarrowMax = 160;
 #define CDN_NARROW_LENGTHS(X) X(64) X(128) X(256)
-static bool y_narrow(int len, long ncols) {
+#define CDN_NARROW_Y_LENGTHS(X) CDN_NARROW_LENGTHS(X) X(2048)
+// slabs: of the launch (planes)
+static bool y_narrow(int len, long ncols, long slabs) {
+  if (len == 2048) return (ncols + kNarrowCols - 1) / kNarrowCols * slabs >= 1024;
   return len == 64 || len == 256 || (len == 128 && ncols <= kNarrowMax);
 }
 static bool z_narrow(int len, long ncols) {
@@ -291,7 +300,7 @@ static ColRun col_run(int len, long ncols, bool narrow) {
 
 void fft_prepare_cols(int len, long ncols, bool z) {
   FftVariant v;
-  if (fft_get_variant(len, &v) || (z ? z_narrow(len, ncols) : y_narrow(len, ncols))) return;
+  if (fft_get_variant(len, &v) || (z ? z_narrow(len, ncols) : y_narrow(len, ncols, 1))) return;
   if (!fft_balanced_cols(len, ncols, &v)) return;
   // compile and load (grid 0: no launch) before any stream capture
   for (JitKernel k : {JK_COL_F, JK_COL_I, JK_Z_FILTER, JK_Z_FILTER_RA}) jit_launch(len, k, 0, 1, nullptr, nullptr, v);
@@ -302,7 +311,7 @@ void launch_col_fft(int len, int inverse, hipStream_t st, float2* S, long ncols,
   // a slab's rows by 32-bit offsets (always the case for y transforms: at
   // most 16384 rows of 8208 columns)
   const bool buf = (double)len * (double)line_stride * 8.0 < 2147483648.0;
-  const ColRun run = col_run(len, ncols, buf && y_narrow(len, ncols));
+  const ColRun run = col_run(len, ncols, buf && y_narrow(len, ncols, n_outer));
   const CShape cs = run.cs;
   long ntiles = (ncols + cs.L - 1) / cs.L;
   const unsigned grid = grid1(ntiles * n_outer);
@@ -320,7 +329,7 @@ void launch_col_fft(int len, int inverse, hipStream_t st, float2* S, long ncols,
     hipLaunchKernelGGL(k, dim3(grid), dim3(cs.THREADS), 0, st, S, ncols, line_stride, outer_stride, ntiles, sp, tw); \
     break;                                                                                                           \
   }
-      CDN_NARROW_LENGTHS(CDN_CASE)
+      CDN_NARROW_Y_LENGTHS(CDN_CASE)
 #undef CDN_CASE
     }
   } else {
@@ -392,7 +401,8 @@ void launch_z_filter(int nz, hipStream_t st, float2* S, long ncols, long line_st
   CDN_HIP(hipGetLastError());
 }
 
-long y_tile_cols(int len, long ncols) { return y_narrow(len, ncols) ? kNarrowCols : c_shape(len).L; }
+// (of many stacks: 2048-point columns in their own width)
+long y_tile_cols(int len, long ncols) { return y_narrow(len, ncols, 0) ? kNarrowCols : c_shape(len).L; }
 long z_tile_cols(int len, long ncols) { return z_narrow(len, ncols) ? kNarrowCols : c_shape(len).L; }
 
 void fft_prepare_ragged(int len) {

@@ -225,6 +225,8 @@ constexpr int kCTptOverride[] = {CDN_CTPT_OVERRIDE};
 constexpr CShape c_shape(int N, int cols = -1, int tpt = -1) {
   CShape s{};
   s.TPT = tpt > 0 ? tpt : lookup_override(kCTptOverride, N) > 0 ? lookup_override(kCTptOverride, N) : tpt_col(N);
+  // a width that would need more than 1024 threads: half as many per column
+  if (tpt <= 0 && cols > 0 && cols * s.TPT > 1024 && s.TPT % 2 == 0 && plan_exact(N, s.TPT / 2)) s.TPT /= 2;
   s.L = lc_for(N, s.TPT, cols);
   s.THREADS = s.TPT * s.L;
   s.E = N / s.TPT;

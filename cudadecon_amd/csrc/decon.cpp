@@ -305,6 +305,7 @@ void RLEngine::iterate(int n, int k0, bool seeded, hipStream_t st, double* lambd
   const float2* twx = fft.twx.as<float2>();
   const float2* twz = fft.twz.as<float2>();
   double* lamd = lam.as<double>();
+  const bool cached = spec_cached(sizeof(float2) * (size_t)fft.nspec * nstacks);
 
   std::vector<hipEvent_t> ev;
   std::vector<int> evpass;
@@ -334,26 +335,27 @@ void RLEngine::iterate(int n, int k0, bool seeded, hipStream_t st, double* lambd
       mode = XIN_PLAIN;
       yv = cur;
     }
-    launch_x_r2c(fft.nx, st, cur, prev, y.as<float>(), lamk, mode, S, rows, fft.pitch, twx, stack_rows);
+    launch_x_r2c(fft.nx, st, cur, prev, y.as<float>(), lamk, mode, S, rows, fft.pitch, twx, stack_rows,
+                 nullptr, 0, cached);
     mark(PASS_XR2C);
     for (int f = 0; f < 2; ++f) {
       // the y transforms see the stacks as nz nstacks slabs
       launch_col_fft(fft.ny, 0, st, S, fft.nxh, fft.pitch, (long)fft.ny * fft.pitch, (long)fft.nz * nstacks,
-                     fft.twy.as<float2>(), op.sup);
+                     fft.twy.as<float2>(), op.sup, cached);
       mark(PASS_YFWD);
       launch_z_filter(fft.nz, st, S, fft.nxh, (long)fft.ny * fft.pitch, fft.pitch, fft.ny, f, op, twz, nstacks,
-                      fft.nspec);
+                      fft.nspec, cached);
       mark(PASS_ZFILT);
       launch_col_fft(fft.ny, 1, st, S, fft.nxh, fft.pitch, (long)fft.ny * fft.pitch, (long)fft.nz * nstacks,
-                     fft.twy.as<float2>(), op.sup);
+                     fft.twy.as<float2>(), op.sup, cached);
       mark(PASS_YINV);
       if (f == 0) {
-        launch_x_lrcore(fft.nx, st, S, raw.as<float>(), rows, fft.pitch, twx, eps);
+        launch_x_lrcore(fft.nx, st, S, raw.as<float>(), rows, fft.pitch, twx, eps, cached);
         mark(PASS_XLR);
       }
     }
     nb_part = launch_x_update(fft.nx, st, S, yv, prev, g.as<float>(), part.as<double>(), k >= 1, rows, fft.pitch,
-                              twx) /
+                              twx, cached) /
               nstacks;
     mark(PASS_XUPD);
     std::swap(cur, prev);

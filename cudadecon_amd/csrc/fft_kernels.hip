@@ -4,6 +4,7 @@
 #include "common.hpp"
 #include "fft_kernels_dev.hpp"
 #include "fft_kernels.hpp"
+#include "fft_kernels_cached.hpp"
 #include "jit.hpp"
 
 #include <algorithm>
@@ -18,9 +19,6 @@ namespace cdn {
 // ---------------------------------------------------------------------------
 // host side: length dispatch
 // ---------------------------------------------------------------------------
-#define CDN_FFT_LENGTHS(X) \
-  X(64) X(96) X(128) X(192) X(256) X(384) X(512) X(768) X(810) X(1024) X(2048)
-
 bool fft_length_precompiled(int n) {
   switch (n) {
 #define CDN_CASE(N) \
@@ -111,7 +109,7 @@ void fft_clear_variants() {
 
 void launch_x_r2c(int nx, hipStream_t st, const float* X, const float* Xp, float* Y, const double* lam, int mode,
                   float2* S, long rows, long pitch, const float2* tw, long stack_rows, const long* row_starts,
-                  int nstk) {
+                  int nstk, bool cached) {
   FftVariant tv;
   const bool tuned = fft_get_variant(nx, &tv);
   const XShape xs = x_shape(nx, tuned ? tv.xthreads : -1, XK_R2C);
@@ -124,6 +122,9 @@ void launch_x_r2c(int nx, hipStream_t st, const float* X, const float* Xp, float
   void* args[] = {&X, &Xp, &Y, &lam, &mode, &S, &rows, &pitch, &stack_rows, &row_starts, &nstk, &tw};
   if (tuned) {
     jit_launch(nx, jk, grid, xs.THREADS, st, args, tv);
+  } else if (auto* k = cached && !ragged ? cached_x_r2c(nx) : nullptr) {
+    hipLaunchKernelGGL(k, dim3(grid), dim3(xs.THREADS), 0, st, X, Xp, Y, lam, mode, S, rows, pitch, stack_rows,
+                       row_starts, nstk, tw);
   } else {
     switch (nx) {
 #define CDN_CASE(N)                                                                                            \
@@ -168,7 +169,7 @@ void launch_x_c2r(int nx, hipStream_t st, const float2* S, float* out, long rows
 }
 
 void launch_x_lrcore(int nx, hipStream_t st, float2* S, const float* raw, long rows, long pitch, const float2* tw,
-                     float eps) {
+                     float eps, bool cached) {
   FftVariant tv;
   const bool tuned = fft_get_variant(nx, &tv);
   const XShape xs = x_shape(nx, tuned ? tv.xthreads : -1, XK_LR);
@@ -176,6 +177,8 @@ void launch_x_lrcore(int nx, hipStream_t st, float2* S, const float* raw, long r
   void* args[] = {&S, &raw, &rows, &pitch, &tw, &eps};
   if (tuned) {
     jit_launch(nx, JK_X_LRCORE, grid, xs.THREADS, st, args, tv);
+  } else if (auto* k = cached ? cached_x_lrcore(nx) : nullptr) {
+    hipLaunchKernelGGL(k, dim3(grid), dim3(xs.THREADS), 0, st, S, raw, rows, pitch, tw, eps);
   } else {
     switch (nx) {
 #define CDN_CASE(N)                                                              \
@@ -207,7 +210,7 @@ long x_update_rows_per_block(int nx) {
 }
 
 int launch_x_update(int nx, hipStream_t st, const float2* S, const float* Y, float* Xout, float* G, double* part,
-                    int dots, long rows, long pitch, const float2* tw) {
+                    int dots, long rows, long pitch, const float2* tw, bool cached) {
   FftVariant tv;
   const bool tuned = fft_get_variant(nx, &tv);
   const XShape xs = x_shape(nx, tuned ? tv.xthreads : -1);
@@ -215,6 +218,8 @@ int launch_x_update(int nx, hipStream_t st, const float2* S, const float* Y, flo
   void* args[] = {&S, &Y, &Xout, &G, &part, &dots, &rows, &pitch, &tw};
   if (tuned) {
     jit_launch(nx, JK_X_UPDATE, grid1(nb), xs.THREADS, st, args, tv);
+  } else if (auto* k = cached ? cached_x_update(nx) : nullptr) {
+    hipLaunchKernelGGL(k, dim3(grid1(nb)), dim3(xs.THREADS), 0, st, S, Y, Xout, G, part, dots, rows, pitch, tw);
   } else {
     switch (nx) {
 #define CDN_CASE(N)                                                                                        \
@@ -269,10 +274,7 @@ bool fft_balanced_cols(int len, long ncols, FftVariant* v) {
 // lines: 0.693 -> 0.632 ms at 96 x 2048 x 2048, 0.180 -> 0.177 at
 // 64 x 2048 x 768 (1600 workgroups), but 0.0425 -> 0.0477 at 32 x 2048 x 256 (288
 // workgroups, a second round of 32), so from 4 rounds of 256 workgroups on.
-constexpr int kNarrowCols = 16;
 constexpr long kNarrowMax = 160;
-#define CDN_NARROW_LENGTHS(X) X(64) X(128) X(256)
-#define CDN_NARROW_Y_LENGTHS(X) CDN_NARROW_LENGTHS(X) X(2048)
 // slabs: of the launch (planes)
 static bool y_narrow(int len, long ncols, long slabs) {
   if (len == 2048) return (ncols + kNarrowCols - 1) / kNarrowCols * slabs >= 1024;
@@ -307,7 +309,7 @@ void fft_prepare_cols(int len, long ncols, bool z) {
 }
 
 void launch_col_fft(int len, int inverse, hipStream_t st, float2* S, long ncols, long line_stride,
-                    long outer_stride, long n_outer, const float2* tw, const OtfSupport& sup) {
+                    long outer_stride, long n_outer, const float2* tw, const OtfSupport& sup, bool cached) {
   // a slab's rows by 32-bit offsets (always the case for y transforms: at
   // most 16384 rows of 8208 columns)
   const bool buf = (double)len * (double)line_stride * 8.0 < 2147483648.0;
@@ -321,6 +323,8 @@ void launch_col_fft(int len, int inverse, hipStream_t st, float2* S, long ncols,
   const JitKernel jk = inverse ? (buf ? JK_COL_I : JK_COL_IW) : (buf ? JK_COL_F : JK_COL_FW);
   if (run.jit) {
     jit_launch(len, jk, grid, cs.THREADS, st, args, run.v);
+  } else if (auto* k = cached && buf ? cached_col(len, inverse != 0, run.narrow) : nullptr) {
+    hipLaunchKernelGGL(k, dim3(grid), dim3(cs.THREADS), 0, st, S, ncols, line_stride, outer_stride, ntiles, sp, tw);
   } else if (run.narrow) {
     switch (len) {
 #define CDN_CASE(N)                                                                                                  \
@@ -357,7 +361,7 @@ static bool z_buf(const CShape& cs, long line_stride) {
 bool z_ragged_buf(int nz, long line_stride) { return z_buf(c_shape(nz), line_stride); }
 
 void launch_z_filter(int nz, hipStream_t st, float2* S, long ncols, long line_stride, long outer_stride, long ny,
-                     int conj, const OtfParams& otf, const float2* tw, int nstacks, long stack_stride) {
+                     int conj, const OtfParams& otf, const float2* tw, int nstacks, long stack_stride, bool cached) {
   const ColRun run = col_run(nz, ncols, z_narrow(nz, ncols) && z_buf(c_shape(nz), line_stride));
   const CShape cs = run.cs;
   long ntiles = (ncols + cs.L - 1) / cs.L;
@@ -370,6 +374,9 @@ void launch_z_filter(int nz, hipStream_t st, float2* S, long ncols, long line_st
   const JitKernel jk = ra ? (buf ? JK_Z_FILTER_RA : JK_Z_FILTER_RA_W) : (buf ? JK_Z_FILTER : JK_Z_FILTER_W);
   if (run.jit) {
     jit_launch(nz, jk, grid, cs.THREADS, st, args, run.v);
+  } else if (auto* k = cached && buf ? cached_z_filter(nz, ra, run.narrow) : nullptr) {
+    hipLaunchKernelGGL(k, dim3(grid), dim3(cs.THREADS), 0, st, S, ncols, line_stride, outer_stride, ntiles, ny,
+                       stack_stride, conj, op, tw);
   } else if (run.narrow) {
     switch (nz) {
 #define CDN_CASE(N)                                                                                             \

@@ -25,24 +25,36 @@ void fft_prepare_length(int n);
 int fft_twiddle_count(int n);
 void fft_twiddles(int n, float2* out);
 
+// Whether an iteration's passes should keep a spectrum of `bytes` in the
+// memory-side cache (256 MB): `cached` of the launchers below, which then run
+// the kernels that access it with cached instructions (real volumes stream as
+// before; lengths without built-in kernels and tuned shapes ignore it).  Each
+// pass then finds the spectrum where the one before left it.  ms per iteration,
+// streaming -> cached: 64 x 512 x 512 (69 MB) 0.329 -> 0.306, 128 x 512 x 512
+// (138 MB) 0.567 -> 0.517, 64 x 768 x 768 (151 MB) 0.687 -> 0.595, 192 x 512 x 512
+// (208 MB) 0.853 -> 0.786, 48 stacks of 64 x 128 x 128 (252 MB) 0.884 -> 0.777;
+// 256 x 512 x 512 (277 MB) 1.079 -> 1.058.  Small spectra stay streaming:
+// 64 x 256 x 256 (19 MB) 0.1195 -> 0.129.
+constexpr bool spec_cached(size_t bytes) { return bytes >= (32UL << 20) && bytes <= (256UL << 20); }
+
 // R2C along x of row pairs with the prediction fused in; writes S.  Rows
 // come in stacks of stack_rows (even; 0: one stack), stack s using the
 // factor lam[4 s]; or, with row_starts (device, nstk ascending even rows,
 // the first 0), in stacks of different heights.
 void launch_x_r2c(int nx, hipStream_t st, const float* X, const float* Xp, float* Y, const double* lam,
                   int mode, float2* S, long rows, long pitch, const float2* tw, long stack_rows = 0,
-                  const long* row_starts = nullptr, int nstk = 0);
+                  const long* row_starts = nullptr, int nstk = 0, bool cached = false);
 // plain C2R along x (ignores imag of kx = 0 and kx = nx/2).
 void launch_x_c2r(int nx, hipStream_t st, const float2* S, float* out, long rows, long pitch,
                   const float2* tw);
 // C2R along x -> LRcore with raw -> R2C along x, in place on S.
 void launch_x_lrcore(int nx, hipStream_t st, float2* S, const float* raw, long rows, long pitch,
-                     const float2* tw, float eps);
+                     const float2* tw, float eps, bool cached = false);
 // C2R along x -> X = max(C Y, 0), G_new = X - Y written over G; if dots:
 // per-block partial sums of G_new.G_old and G_old.G_old (FP32 products,
 // FP64 sums) into part[2*block..].  Returns the number of blocks launched.
 int launch_x_update(int nx, hipStream_t st, const float2* S, const float* Y, float* Xout, float* G,
-                    double* part, int dots, long rows, long pitch, const float2* tw);
+                    double* part, int dots, long rows, long pitch, const float2* tw, bool cached = false);
 int x_update_blocks(int nx, long rows);
 // rows per x-update workgroup of the launch shape in use for nx
 long x_update_rows_per_block(int nx);
@@ -78,12 +90,13 @@ constexpr OtfSupport kNoSupport{-1.f, 0.f, 0.f};
 // y transforms around a z filter, the support of its OTF (the rows outside it
 // are not stored by the forward and taken as zero by the inverse transform).
 void launch_col_fft(int len, int inverse, hipStream_t st, float2* S, long ncols, long line_stride,
-                    long outer_stride, long n_outer, const float2* tw, const OtfSupport& sup = kNoSupport);
+                    long outer_stride, long n_outer, const float2* tw, const OtfSupport& sup = kNoSupport,
+                    bool cached = false);
 // z forward -> x H (or conj H) / N -> z inverse; slab index = ky, for
 // nstacks spectra stack_stride complex elements apart.
 void launch_z_filter(int nz, hipStream_t st, float2* S, long ncols, long line_stride, long outer_stride,
                      long ny, int conj, const OtfParams& otf, const float2* tw, int nstacks = 1,
-                     long stack_stride = 0);
+                     long stack_stride = 0, bool cached = false);
 
 // Column passes spanning stacks of different shapes: one launch for every
 // stack whose transform length is `len`, segs (device) one per stack with

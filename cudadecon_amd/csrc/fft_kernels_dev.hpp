@@ -24,7 +24,10 @@ namespace cdn {
 
 // Non-temporal policy per kernel family (measured at 256 x 1024 x 1024):
 // x passes and the z filter stream both ways; plain y/z column transforms
-// keep cached loads and stream their stores.
+// keep cached loads and stream their stores.  CDN_SPEC_CACHED: the spectrum is
+// read and written with cached instructions throughout, for spectra that fit
+// the memory-side cache (see spec_cached in fft_kernels.hpp); these kernels
+// live in a namespace of their own.
 #ifndef CDN_NT_X
 #define CDN_NT_X 1
 #endif
@@ -37,8 +40,27 @@ namespace cdn {
 #ifndef CDN_NT_COL_STORE
 #define CDN_NT_COL_STORE 1
 #endif
-constexpr bool NTX = CDN_NT_X != 0, NTZ = CDN_NT_Z != 0;
-constexpr bool NTCL = CDN_NT_COL_LOAD != 0, NTCS = CDN_NT_COL_STORE != 0;
+#ifndef CDN_SPEC_CACHED
+#define CDN_SPEC_CACHED 0
+#endif
+#ifndef __HIPCC_RTC__
+#if CDN_SPEC_CACHED
+inline namespace spec_cached_kernels {
+#else
+inline namespace spec_stream_kernels {
+#endif
+#endif
+// NTX: real volumes of the x passes, NTXS: their spectrum rows
+constexpr bool NTX = CDN_NT_X != 0, NTXS = CDN_NT_X != 0 && !CDN_SPEC_CACHED;
+constexpr bool NTZ = CDN_NT_Z != 0 && !CDN_SPEC_CACHED;
+constexpr bool NTCL = CDN_NT_COL_LOAD != 0, NTCS = CDN_NT_COL_STORE != 0 && !CDN_SPEC_CACHED;
+
+// Lengths with built-in kernels, and those with column tiles of 16
+#define CDN_FFT_LENGTHS(X) \
+  X(64) X(96) X(128) X(192) X(256) X(384) X(512) X(768) X(810) X(1024) X(2048)
+#define CDN_NARROW_LENGTHS(X) X(64) X(128) X(256)
+#define CDN_NARROW_Y_LENGTHS(X) CDN_NARROW_LENGTHS(X) X(2048)
+constexpr int kNarrowCols = 16;
 
 // ---------------------------------------------------------------------------
 // Per-length launch configuration
@@ -300,25 +322,25 @@ template <int STEP> struct RowsPtr {
   long pitch;
   bool v0, v1;
   __device__ __forceinline__ void load(int m, bool on, float2& A, float2& B) const {
-    A = on && v0 ? ld_stream<NTX>(S + m * STEP) : make_float2(0.f, 0.f);
-    B = on && v1 ? ld_stream<NTX>(S + pitch + m * STEP) : make_float2(0.f, 0.f);
+    A = on && v0 ? ld_stream<NTXS>(S + m * STEP) : make_float2(0.f, 0.f);
+    B = on && v1 ? ld_stream<NTXS>(S + pitch + m * STEP) : make_float2(0.f, 0.f);
   }
   __device__ __forceinline__ void store(int m, bool on, float2 A, float2 B) const {
     if (!on) return;
-    if (v0) st_stream<NTX>(S + m * STEP, A);
-    if (v1) st_stream<NTX>(S + pitch + m * STEP, B);
+    if (v0) st_stream<NTXS>(S + m * STEP, A);
+    if (v1) st_stream<NTXS>(S + pitch + m * STEP, B);
   }
 };
 template <int STEP> struct RowsBuf {
   SlabBuf b;
   int off, pitch8;  // bytes: of element p of the first row, per row
   __device__ __forceinline__ void load(int m, bool on, float2& A, float2& B) const {
-    A = b.template load<NTX>(on ? off : kNoRow, m * STEP * 8);
-    B = b.template load<NTX>(on ? off : kNoRow, m * STEP * 8 + pitch8);
+    A = b.template load<NTXS>(on ? off : kNoRow, m * STEP * 8);
+    B = b.template load<NTXS>(on ? off : kNoRow, m * STEP * 8 + pitch8);
   }
   __device__ __forceinline__ void store(int m, bool on, float2 A, float2 B) const {
-    b.template store<NTX>(on ? off : kNoRow, m * STEP * 8, A);
-    b.template store<NTX>(on ? off : kNoRow, m * STEP * 8 + pitch8, B);
+    b.template store<NTXS>(on ? off : kNoRow, m * STEP * 8, A);
+    b.template store<NTXS>(on ? off : kNoRow, m * STEP * 8 + pitch8, B);
   }
 };
 
@@ -945,4 +967,7 @@ __global__ void __launch_bounds__((CCfg<N, COLS>::THREADS))
   } while (it < total);
 }
 
+#ifndef __HIPCC_RTC__
+}  // inline namespace
+#endif
 }  // namespace cdn

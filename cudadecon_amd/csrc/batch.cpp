@@ -298,6 +298,7 @@ void Batch::enqueue_partition(const Partition& P, hipStream_t st, int iters, hip
   float* c = a_xa.as<float>();
   float* pv = a_xb.as<float>();
   float2* spec = a_spec.as<float2>();
+  const bool cached = spec_cached(a_spec.bytes);
   for (int k = 0; k < iters; ++k) {
     double* lamk = g_lam.as<double>() + 4 * (size_t)n * k;
     if (k >= 2)
@@ -306,29 +307,30 @@ void Batch::enqueue_partition(const Partition& P, hipStream_t st, int iters, hip
     const int mode = k >= 2 ? XIN_PRED : XIN_PLAIN;
     for (const XGroup& g : P.xg)
       launch_x_r2c(g.nx, st, c + g.voff, pv + g.voff, a_y.as<float>() + g.voff, lamk + 4 * g.first, mode,
-                   spec + g.soff, g.rows, g.pitch, g.tw, 0, g.row_starts.as<long>(), g.count);
+                   spec + g.soff, g.rows, g.pitch, g.tw, 0, g.row_starts.as<long>(), g.count, cached);
     CDN_HIP(hipEventRecord(mark, st));
     for (int f = 0; f < 2; ++f) {
       for (const ColGroup& g : P.yg)
-        launch_col_ragged(g.len, 0, st, g.segs.as<ColSeg>(), g.nseg, g.total, g.cols, g.tw, grid_cap);
+        launch_col_ragged(g.len, 0, st, g.segs.as<ColSeg>(), g.nseg, g.total, g.cols, g.tw, grid_cap, cached);
       CDN_HIP(hipEventRecord(mark, st));
       for (const ColGroup& g : P.zg)
         launch_z_ragged(g.len, st, g.segs.as<ZSeg>(), g.nseg, g.total, g.cols, f, g.tw, grid_cap, g.ra,
-                        g.buf);
+                        g.buf, cached);
       CDN_HIP(hipEventRecord(mark, st));
       for (const ColGroup& g : P.yg)
-        launch_col_ragged(g.len, 1, st, g.segs.as<ColSeg>(), g.nseg, g.total, g.cols, g.tw, grid_cap);
+        launch_col_ragged(g.len, 1, st, g.segs.as<ColSeg>(), g.nseg, g.total, g.cols, g.tw, grid_cap, cached);
       CDN_HIP(hipEventRecord(mark, st));
       if (f == 0) {
         for (const XGroup& g : P.xg)
-          launch_x_lrcore(g.nx, st, spec + g.soff, a_raw.as<float>() + g.voff, g.rows, g.pitch, g.tw, eps);
+          launch_x_lrcore(g.nx, st, spec + g.soff, a_raw.as<float>() + g.voff, g.rows, g.pitch, g.tw, eps,
+                          cached);
         CDN_HIP(hipEventRecord(mark, st));
       }
     }
     const float* yv = k >= 2 ? a_y.as<float>() : c;
     for (const XGroup& g : P.xg) {
       const int nb = launch_x_update(g.nx, st, spec + g.soff, yv + g.voff, pv + g.voff, a_g.as<float>() + g.voff,
-                                     g_part.as<double>() + 2 * g.part0, k >= 1, g.rows, g.pitch, g.tw);
+                                     g_part.as<double>() + 2 * g.part0, k >= 1, g.rows, g.pitch, g.tw, cached);
       if (nb != g.nb) fail("batch: the x-update launch shape changed under the grouped schedule");
     }
     std::swap(c, pv);

@@ -122,7 +122,7 @@ void launch_x_r2c(int nx, hipStream_t st, const float* X, const float* Xp, float
   void* args[] = {&X, &Xp, &Y, &lam, &mode, &S, &rows, &pitch, &stack_rows, &row_starts, &nstk, &tw};
   if (tuned) {
     jit_launch(nx, jk, grid, xs.THREADS, st, args, tv);
-  } else if (auto* k = cached && !ragged ? cached_x_r2c(nx) : nullptr) {
+  } else if (auto* k = cached ? cached_x_r2c(nx, ragged) : nullptr) {
     hipLaunchKernelGGL(k, dim3(grid), dim3(xs.THREADS), 0, st, X, Xp, Y, lam, mode, S, rows, pitch, stack_rows,
                        row_starts, nstk, tw);
   } else {
@@ -435,15 +435,16 @@ static auto col_ragged_n(bool inv, bool pers) {
 }
 
 void launch_col_ragged(int len, int inverse, hipStream_t st, const ColSeg* segs, int nseg, long total, long cols,
-                       const float2* tw, long grid_cap) {
+                       const float2* tw, long grid_cap, bool cached) {
   if (total <= 0) return;
   const bool narrow = cols != c_shape(len).L;
   const CShape cs = c_shape(len, narrow ? (int)cols : -1);
   const unsigned grid = ragged_grid(total, grid_cap);
   const bool inv = inverse != 0, pers = grid < total;
   void* args[] = {&segs, &nseg, &total, &tw};
-  void (*k)(const ColSeg*, int, long, const float2*) = nullptr;
-  if (narrow) {
+  ColRaggedKernel* k = cached && !pers ? cached_col_ragged(len, inv, narrow) : nullptr;
+  if (k) {
+  } else if (narrow) {
     switch (len) {
 #define CDN_CASE(N) \
   case N: k = col_ragged_n<N, kNarrowCols>(inv, pers); break;
@@ -477,15 +478,16 @@ static auto z_ragged_n(bool pers, bool ra, bool buf) {
 }
 
 void launch_z_ragged(int nz, hipStream_t st, const ZSeg* segs, int nseg, long total, long cols, int conj,
-                     const float2* tw, long grid_cap, bool ra, bool buf) {
+                     const float2* tw, long grid_cap, bool ra, bool buf, bool cached) {
   if (total <= 0) return;
   const bool narrow = cols != c_shape(nz).L;
   const CShape cs = c_shape(nz, narrow ? (int)cols : -1);
   const unsigned grid = ragged_grid(total, buf ? grid_cap : 0);
   const bool pers = grid < total;
   void* args[] = {&segs, &nseg, &total, &conj, &tw};
-  void (*k)(const ZSeg*, int, long, int, const float2*) = nullptr;
-  if (narrow) {
+  ZRaggedKernel* k = cached && buf && !pers ? cached_z_ragged(nz, ra, narrow) : nullptr;
+  if (k) {
+  } else if (narrow) {
     switch (nz) {
 #define CDN_CASE(N) \
   case N: k = z_ragged_n<N, kNarrowCols>(pers, ra, true); break;

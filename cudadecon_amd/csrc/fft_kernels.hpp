@@ -33,7 +33,8 @@ void fft_twiddles(int n, float2* out);
 // streaming -> cached: 64 x 512 x 512 (69 MB) 0.329 -> 0.306, 128 x 512 x 512
 // (138 MB) 0.567 -> 0.517, 64 x 768 x 768 (151 MB) 0.687 -> 0.595, 192 x 512 x 512
 // (208 MB) 0.853 -> 0.786, 48 stacks of 64 x 128 x 128 (252 MB) 0.884 -> 0.777;
-// 256 x 512 x 512 (277 MB) 1.079 -> 1.058.  Small spectra stay streaming:
+// 256 x 512 x 512 (277 MB) 1.079 -> 1.058; 24 uneven stacks in one graph
+// (156 MB) 0.96 -> 0.87.  Small spectra stay streaming:
 // 64 x 256 x 256 (19 MB) 0.1195 -> 0.129.
 constexpr bool spec_cached(size_t bytes) { return bytes >= (32UL << 20) && bytes <= (256UL << 20); }
 
@@ -108,11 +109,12 @@ long z_tile_cols(int len, long ncols);
 // built in will use (no GPU work; call before any stream capture)
 void fft_prepare_ragged(int len);
 void launch_col_ragged(int len, int inverse, hipStream_t st, const ColSeg* segs, int nseg, long total,
-                       long cols, const float2* tw, long grid_cap = 0);
+                       long cols, const float2* tw, long grid_cap = 0, bool cached = false);
 // ra: every segment's OTF is rotationally averaged (the kernel kind the
 // one-stack z filter uses for such a table)
 void launch_z_ragged(int nz, hipStream_t st, const ZSeg* segs, int nseg, long total, long cols, int conj,
-                     const float2* tw, long grid_cap = 0, bool ra = false, bool buf = true);
+                     const float2* tw, long grid_cap = 0, bool ra = false, bool buf = true,
+                     bool cached = false);
 // whether a stack's z filter can address its planes (line_stride apart) by
 // 32-bit offsets: buf above, for every segment of the launch
 bool z_ragged_buf(int nz, long line_stride);

@@ -13,10 +13,10 @@ namespace cdn {
       return nullptr;           \
   }
 
-XR2cKernel* cached_x_r2c(int n) {
+XR2cKernel* cached_x_r2c(int n, bool ragged) {
 #define CDN_CASE(N) \
   case N:           \
-    return k_x_r2c<N, false>;
+    return ragged ? k_x_r2c<N, true> : k_x_r2c<N, false>;
   CDN_PICK(CDN_FFT_LENGTHS, CDN_CASE)
 #undef CDN_CASE
 }
@@ -63,6 +63,36 @@ ZFilterKernel* cached_z_filter(int n, bool ra, bool narrow) {
 #define CDN_CASE(N) \
   case N:           \
     return ra ? k_z_filter<N, ZF_RA, true> : k_z_filter<N, ZF_ANY, true>;
+  CDN_PICK(CDN_FFT_LENGTHS, CDN_CASE)
+#undef CDN_CASE
+}
+
+ColRaggedKernel* cached_col_ragged(int n, bool inverse, bool narrow) {
+  if (narrow) {
+#define CDN_CASE(N) \
+  case N:           \
+    return inverse ? k_col_ragged<N, true, false, kNarrowCols> : k_col_ragged<N, false, false, kNarrowCols>;
+    CDN_PICK(CDN_NARROW_LENGTHS, CDN_CASE)
+#undef CDN_CASE
+  }
+#define CDN_CASE(N) \
+  case N:           \
+    return inverse ? k_col_ragged<N, true, false> : k_col_ragged<N, false, false>;
+  CDN_PICK(CDN_FFT_LENGTHS, CDN_CASE)
+#undef CDN_CASE
+}
+
+ZRaggedKernel* cached_z_ragged(int n, bool ra, bool narrow) {
+  if (narrow) {
+#define CDN_CASE(N) \
+  case N:           \
+    return ra ? k_z_ragged<N, false, ZF_RA, true, kNarrowCols> : k_z_ragged<N, false, ZF_ANY, true, kNarrowCols>;
+    CDN_PICK(CDN_NARROW_LENGTHS, CDN_CASE)
+#undef CDN_CASE
+  }
+#define CDN_CASE(N) \
+  case N:           \
+    return ra ? k_z_ragged<N, false, ZF_RA> : k_z_ragged<N, false, ZF_ANY>;
   CDN_PICK(CDN_FFT_LENGTHS, CDN_CASE)
 #undef CDN_CASE
 }

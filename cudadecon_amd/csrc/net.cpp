@@ -14,7 +14,6 @@ namespace {
 constexpr int WG_CHUNKS = 512;
 constexpr int wg_chunks(int l) { return NET_CIN[l] * NET_COUT[l] > 1024 ? WG_CHUNKS / 2 : WG_CHUNKS; }
 constexpr int WG_CHUNKS_IN1 = 1024;  // first layer
-constexpr int CS_BLOCKS = 256;      // bias-gradient partial rows
 
 struct SplitMix {
   uint64_t s;
@@ -122,8 +121,7 @@ void WarmNet::geometry(int nb, int nz, int ny, int nx, bool training) {
     gP1.ensure(h * n2 * 16);
     g1.ensure(h * n1 * 16);
     hpart.ensure(sizeof(float) * 18 * (size_t)net_head_blocks(L1));
-    cpart.ensure(sizeof(float) * 64 * CS_BLOCKS);
-    wpart.ensure(sizeof(float) * std::max(27L * 64 * 32 * wg_chunks(2), 27L * 16 * WG_CHUNKS_IN1));
+    wpart.ensure(sizeof(float) * std::max((27L * 32 + 1) * 64 * wg_chunks(2), 28L * 16 * WG_CHUNKS_IN1));
     loss.ensure(sizeof(float) * 4);
   }
 }
@@ -174,9 +172,8 @@ void WarmNet::backward(hipStream_t st, const float* raw, const float* tgt, float
 
   auto wgrad = [&](int l, const bf16_t* in, const bf16_t* gr, const Vol& v) {
     const int rows = net_wgrad(st, NET_CIN[l], NET_COUT[l], in, gr, v, wg_chunks(l), wpart.as<float>());
-    net_reduce_rows(st, wpart.as<float>(), rows, 27L * NET_CIN[l] * NET_COUT[l], g + w_off[l]);
-    net_chan_sum(st, NET_COUT[l], gr, vox(v), CS_BLOCKS, cpart.as<float>());
-    net_reduce_rows(st, cpart.as<float>(), CS_BLOCKS, NET_COUT[l], g + b_off[l]);
+    // the biases follow the weights
+    net_reduce_rows(st, wpart.as<float>(), rows, (27L * NET_CIN[l] + 1) * NET_COUT[l], g + w_off[l]);
   };
   // conv5 (a2 -> d2)
   net_grad_dec(st, 16, d2.as<bf16_t>(), nullptr, dO, wh, g5.as<bf16_t>(), L2);
@@ -197,9 +194,7 @@ void WarmNet::backward(hipStream_t st, const float* raw, const float* tgt, float
   // conv1 (u -> e1); e1 also feeds the head directly
   net_grad_enc(st, 16, e1.as<bf16_t>(), nullptr, dO, wh, gP1.as<bf16_t>(), g1.as<bf16_t>(), L1);
   const int rows1 = net_wgrad_in1(st, raw, inv_s.as<float>(), g1.as<bf16_t>(), L1, WG_CHUNKS_IN1, wpart.as<float>());
-  net_reduce_rows(st, wpart.as<float>(), rows1, 27L * 16, g + w_off[0]);
-  net_chan_sum(st, 16, g1.as<bf16_t>(), vox(L1), CS_BLOCKS, cpart.as<float>());
-  net_reduce_rows(st, cpart.as<float>(), CS_BLOCKS, 16, g + b_off[0]);
+  net_reduce_rows(st, wpart.as<float>(), rows1, 28L * 16, g + w_off[0]);
 }
 
 void WarmNet::adam(hipStream_t st, float lr) {

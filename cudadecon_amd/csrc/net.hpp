@@ -34,7 +34,7 @@ struct WarmNet {
   DevBuf inv_s, sum_part;
   DevBuf e1, p1, e2, p2, e3, d3, a2, d2;
   DevBuf dout, g5, gA2, g4, gE3, g3, gP2, g2, gP1, g1;
-  DevBuf hpart, cpart, wpart, loss;
+  DevBuf hpart, wpart, loss;
   // training set (FP32 stacks and targets of one patch shape)
   long ds_count = 0;
   int ds_nz = 0, ds_ny = 0, ds_nx = 0;

@@ -894,38 +894,6 @@ __global__ void k_grad_dec(const bf16_t* __restrict__ d, const bf16_t* __restric
   }
 }
 
-// Per-block channel sums of a [n][C] BF16 tensor (bias gradients):
-// part[block][C].  Threads own a fixed channel group; LDS tree per group.
-template <int C>
-__global__ __launch_bounds__(256) void k_chan_sum(const bf16_t* __restrict__ t, long nvox, float* __restrict__ part) {
-  constexpr int G = C / 8;
-  const int g = threadIdx.x % G;
-  float s[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  const long n = nvox * G;
-  for (long i = blockIdx.x * 256L + threadIdx.x; i < n; i += (long)gridDim.x * 256) {
-    const u32x4 d = *reinterpret_cast<const u32x4*>(t + (i / G) * C + 8 * g);
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      s[2 * k] += lo(d[k]);
-      s[2 * k + 1] += hi(d[k]);
-    }
-  }
-  __shared__ float red[256][9];
-#pragma unroll
-  for (int k = 0; k < 8; ++k) red[threadIdx.x][k] = s[k];
-  __syncthreads();
-  // 256 is a multiple of G: threads tid, tid+G, ... share a channel group
-  for (int stride = 128; stride >= G; stride >>= 1) {
-    if ((int)threadIdx.x < stride)
-#pragma unroll
-      for (int k = 0; k < 8; ++k) red[threadIdx.x][k] += red[threadIdx.x + stride][k];
-    __syncthreads();
-  }
-  if ((int)threadIdx.x < G)
-#pragma unroll
-    for (int k = 0; k < 8; ++k) part[blockIdx.x * (long)C + 8 * threadIdx.x + k] = red[threadIdx.x][k];
-}
-
 // ---------------------------------------------------------------------------
 // Weight gradient: dW[t][ci][co] = sum_v in[v + t][ci] * dPre[v][co].
 // MFMA with K = 32 voxels along x: A = dPre^T (m = co), B = the input
@@ -937,7 +905,12 @@ __global__ __launch_bounds__(256) void k_chan_sum(const bf16_t* __restrict__ t, 
 // the step before stay in a ring of 3) and one gradient row, kept in 3 copies
 // shifted by dx so that every fragment read is aligned.  The next step's rows
 // are loaded into registers before the products of this one.  Wave w of 8
-// takes taps w, w + 8, ... with all channel blocks.
+// takes taps w, w + 8, ... with all channel blocks; "tap" 27, an input of ones,
+// gives the bias gradient (a partial row is 27 cin cout weights, then cout
+// biases, as the parameters lie).  Channel sums of their own read every
+// gradient tensor once more (394 MB) in 10 launches: a step with its uploads at
+// 8 patches of 64 x 128 x 128 took 3.56 ms with them and takes 3.35; the errors
+// to the FP64 sums are the same (5e-8).
 // What bounds it is LDS: 27 (CIN + COUT) / 16 fragment reads of 1 KB per 32
 // voxels, and the transposing 2-byte writes.  Against one wave per tap and
 // chunk of rows (1728 waves) that gathered each fragment by 2-byte global
@@ -978,6 +951,7 @@ __global__ __launch_bounds__(WG_THREADS) void k_wgrad(const bf16_t* __restrict__
   __shared__ __attribute__((aligned(16))) bf16_t ring[3][3][CIN][WGP];  // [dz + 1][row mod 3][ci][x]
   __shared__ __attribute__((aligned(16))) bf16_t gs[3][COUT][WGP];      // [dx + 1][co][x] = g[x - dx]
   const int tid = threadIdx.x, lane = tid & 63, q = lane >> 4, r = lane & 15, wave = tid >> 6;
+  const u32x4 ONES = {0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};
   f32x4 acc[NT][NBO][NBI];
 #pragma unroll
   for (int a = 0; a < NT; ++a)
@@ -1074,6 +1048,12 @@ __global__ __launch_bounds__(WG_THREADS) void k_wgrad(const bf16_t* __restrict__
               for (int p = 0; p < NBI; ++p) acc[a][j][p] = Mfma<32>::run(am, b[p], acc[a][j][p]);
             }
           }
+        } else if (t == 27) {
+          for (int ks = 0; ks < nk; ++ks)
+#pragma unroll
+            for (int j = 0; j < NBO; ++j)
+              acc[a][j][0] = Mfma<32>::run(*reinterpret_cast<const u32x4*>(&gs[1][16 * j + r][8 * q + 32 * ks]), ONES,
+                                           acc[a][j][0]);
         }
       }
       __syncthreads();  // the next step's rows go over these
@@ -1083,8 +1063,14 @@ __global__ __launch_bounds__(WG_THREADS) void k_wgrad(const bf16_t* __restrict__
 #pragma unroll
   for (int a = 0; a < NT; ++a) {
     const int t = wave + a * WG_WAVES;
+    float* row = part + (long)blockIdx.x * (27 * CIN * COUT + COUT);
+    if (t == 27 && r == 0) {
+#pragma unroll
+      for (int j = 0; j < NBO; ++j)
+        *reinterpret_cast<f32x4*>(row + 27 * CIN * COUT + 16 * j + 4 * q) = acc[a][j][0];
+    }
     if (t < 27) {
-      float* dst = part + ((long)blockIdx.x * 27 + t) * CIN * COUT;
+      float* dst = row + (long)t * CIN * COUT;
 #pragma unroll
       for (int j = 0; j < NBO; ++j)
 #pragma unroll
@@ -1094,22 +1080,26 @@ __global__ __launch_bounds__(WG_THREADS) void k_wgrad(const bf16_t* __restrict__
   }
 }
 
-// First layer weight gradient: n runs over the taps (two blocks of 16, taps
-// >= 27 dropped), the input is bf16(raw / s) as in the forward pass.  Staged
-// as above, 128 voxels of x per workgroup and 32 per wave; here the one-channel
-// input has the copies shifted by dx ([x] = u[x + dx]).  Bound by reading the
-// gradient (16 channels of the full-size level, 268 MB at 8 patches of
-// 64 x 128 x 128): 2010 us from 512 waves gathering single values, 132 now.
+// First layer weight gradient: n runs over the taps (two blocks of 16; tap 27
+// is an input of ones, the bias gradient, the rest is dropped), the input is
+// bf16(raw / s) as in the forward pass.  Staged as above, 128 voxels of x per
+// workgroup and 32 per wave; here the one-channel input has the copies shifted
+// by dx ([x] = u[x + dx]).  Bound by reading the gradient (16 channels of the
+// full-size level, 268 MB at 8 patches of 64 x 128 x 128): 2010 us from 512
+// waves gathering single values, 132 now.
 constexpr int W1X = 128, W1P = W1X + 8;
 __global__ __launch_bounds__(256) void k_wgrad_in1(const float* __restrict__ raw, const float* __restrict__ inv_s,
                                                    const bf16_t* __restrict__ gr, Vol v, WgItems wi,
                                                    float* __restrict__ part) {
-  // rows [dz + 1][row mod 3][dx + 1][x]; the last row stays zero (taps >= 27)
-  __shared__ __attribute__((aligned(16))) bf16_t ring[28][W1P];
+  // rows [dz + 1][row mod 3][dx + 1][x]; then ones (tap 27) and zeros (beyond)
+  __shared__ __attribute__((aligned(16))) bf16_t ring[29][W1P];
   __shared__ __attribute__((aligned(16))) bf16_t gs[16][W1P];
   __shared__ __attribute__((aligned(16))) float red[4][32 * 16];
   const int tid = threadIdx.x, lane = tid & 63, q = lane >> 4, r = lane & 15, wave = tid >> 6;
-  for (int i = tid; i < W1P; i += 256) ring[27][i] = 0;
+  for (int i = tid; i < W1P; i += 256) {
+    ring[27][i] = 0x3f80;
+    ring[28][i] = 0;
+  }
   f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
   // the planes' rows in 3 (W1X + 2) loads, 2 per thread
   constexpr int IN_U = 3 * (W1X + 2), IN_N = (IN_U + 255) / 256;
@@ -1168,7 +1158,7 @@ __global__ __launch_bounds__(256) void k_wgrad_in1(const float* __restrict__ raw
       const u32x4 a = *reinterpret_cast<const u32x4*>(&gs[r][32 * wave + 8 * q]);
 #pragma unroll
       for (int p = 0; p < 2; ++p) {
-        const int t = 16 * p + r, row = t < 27 ? (t / 9 * 3 + (y + t / 3 % 3 + 2) % 3) * 3 + t % 3 : 27;
+        const int t = 16 * p + r, row = t < 27 ? (t / 9 * 3 + (y + t / 3 % 3 + 2) % 3) * 3 + t % 3 : t == 27 ? 27 : 28;
         const u32x4 b = *reinterpret_cast<const u32x4*>(&ring[row][32 * wave + 8 * q]);
         acc[p] = Mfma<32>::run(a, b, acc[p]);
       }
@@ -1179,8 +1169,8 @@ __global__ __launch_bounds__(256) void k_wgrad_in1(const float* __restrict__ raw
 #pragma unroll
   for (int p = 0; p < 2; ++p) *reinterpret_cast<f32x4*>(&red[wave][(16 * p + r) * 16 + 4 * q]) = acc[p];
   __syncthreads();
-  for (int i = tid; i < 27 * 16; i += 256)
-    part[(long)blockIdx.x * 27 * 16 + i] = ((red[0][i] + red[1][i]) + red[2][i]) + red[3][i];
+  for (int i = tid; i < 28 * 16; i += 256)
+    part[(long)blockIdx.x * 28 * 16 + i] = ((red[0][i] + red[1][i]) + red[2][i]) + red[3][i];
 }
 
 // out[c] = sum_g part[g][c] in double, in a fixed order: a workgroup takes 64
@@ -1502,13 +1492,6 @@ void net_grad_dec(hipStream_t st, int c, const bf16_t* d, const bf16_t* fine, co
   if (c == 16) hipLaunchKernelGGL(k_grad_dec<16>, dim3(grid), dim3(256), 0, st, d, fine, dout, wh, dpre, coarse);
   else if (c == 32) hipLaunchKernelGGL(k_grad_dec<32>, dim3(grid), dim3(256), 0, st, d, fine, dout, wh, dpre, coarse);
   else fail("net_grad_dec: channels");
-}
-
-void net_chan_sum(hipStream_t st, int c, const bf16_t* t, long nvox, int blocks, float* part) {
-  if (c == 16) hipLaunchKernelGGL(k_chan_sum<16>, dim3(blocks), dim3(256), 0, st, t, nvox, part);
-  else if (c == 32) hipLaunchKernelGGL(k_chan_sum<32>, dim3(blocks), dim3(256), 0, st, t, nvox, part);
-  else if (c == 64) hipLaunchKernelGGL(k_chan_sum<64>, dim3(blocks), dim3(256), 0, st, t, nvox, part);
-  else fail("net_chan_sum: channels");
 }
 
 int net_wgrad(hipStream_t st, int cin, int cout, const bf16_t* in, const bf16_t* g, Vol v, int G, float* part) {

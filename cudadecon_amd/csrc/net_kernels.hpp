@@ -40,8 +40,8 @@ void net_grad_enc(hipStream_t st, int c, const bf16_t* e, const bf16_t* skip, co
                   const bf16_t* dP, bf16_t* dpre, Vol v);
 void net_grad_dec(hipStream_t st, int c, const bf16_t* d, const bf16_t* fine, const float* dout, const float* wh,
                   bf16_t* dpre, Vol coarse);
-void net_chan_sum(hipStream_t st, int c, const bf16_t* t, long nvox, int blocks, float* part);
-// weight gradients in at most G partial rows of 27 cin cout; returns how many
+// weight and bias gradients in at most G partial rows of 27 cin cout + cout
+// (the parameters' order); returns how many
 int net_wgrad(hipStream_t st, int cin, int cout, const bf16_t* in, const bf16_t* g, Vol v, int G, float* part);
 int net_wgrad_in1(hipStream_t st, const float* raw, const float* inv_s, const bf16_t* g, Vol v, int G, float* part);
 void net_reduce_rows(hipStream_t st, const float* part, int rows, long cols, float* out);

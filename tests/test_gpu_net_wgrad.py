@@ -42,3 +42,23 @@ def test_weight_gradients_at_tile_edges(cdn, shape):
         assert np.linalg.norm(g[w] - gb[w]) <= 3e-2 * np.linalg.norm(gb[w]), l
     cos = float(g @ ge / (np.linalg.norm(g) * np.linalg.norm(ge)))
     assert cos >= 0.995
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+def test_bias_gradients_are_the_sums_of_the_backward_tensors(cdn, shape):
+    """The same kernels' 28th tap.  Against the FP64 sum of the very BF16 tensor
+    that the kernel read: a chain of at most 64 products of 32 voxels in FP32 at
+    these sizes, then FP64, so (64 + 32) 2^-24 < 1e-5 of the absolute sum."""
+    print("bias grad", shape, flush=True)
+    rng = np.random.default_rng(8)
+    p = N.he_init(2)
+    w_off, b_off, h, _ = N.layout()
+    p[h:h + 16] = 0.2 * rng.standard_normal(16)
+    raw = rng.gamma(2.0, 50.0, shape).astype(np.float32)
+    tgt = (raw * rng.uniform(0.5, 1.5, shape)).astype(np.float32)
+    net = cdn.WarmNet(params=p.astype(np.float32))
+    _, g = net.loss_grad(raw, tgt)
+    for l in range(5):
+        pre = net.fetch("dPre%d" % (l + 1)).reshape(-1, N.COUT[l]).astype(np.float64)
+        got = g[b_off[l]:b_off[l] + N.COUT[l]]
+        assert np.all(np.abs(got - pre.sum(0)) <= 1e-5 * np.abs(pre).sum(0)), l

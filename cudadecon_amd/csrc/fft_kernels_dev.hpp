@@ -282,7 +282,11 @@ template <int N, int COLS = 0> struct CCfg {
 // leaves one workgroup per CU instead of two (0.393 ms, every row read 0.382,
 // this form 0.357).  Registers of the y transforms: 64 to 2048 points 60-92
 // -> 56-81, of the z filters 92-142 -> 84-126 at 64 to 192 points.
-// Loads past the end return zero and stores there do nothing.
+// The range check is the vector offset's alone: the scalar offset is defined as
+// taking no part in it (and where it did, subtracting it from a length that it
+// exceeds would not help).  So an element past the end must be past it by its
+// vector offset, or have kNoRow there; its load returns zero, its store does
+// nothing.  Scalar offsets stay inside what the vector offset leaves.
 constexpr int kNoRow = -1;  // past every end
 typedef unsigned u2v __attribute__((ext_vector_type(2)));
 struct SlabBuf {
@@ -333,14 +337,14 @@ template <int STEP> struct RowsPtr {
 };
 template <int STEP> struct RowsBuf {
   SlabBuf b;
-  int off, pitch8;  // bytes: of element p of the first row, per row
+  int offA, offB;  // bytes: of element p of the two rows, kNoRow for a row past the last
   __device__ __forceinline__ void load(int m, bool on, float2& A, float2& B) const {
-    A = b.template load<NTXS>(on ? off : kNoRow, m * STEP * 8);
-    B = b.template load<NTXS>(on ? off : kNoRow, m * STEP * 8 + pitch8);
+    A = b.template load<NTXS>(on ? offA : kNoRow, m * STEP * 8);
+    B = b.template load<NTXS>(on ? offB : kNoRow, m * STEP * 8);
   }
   __device__ __forceinline__ void store(int m, bool on, float2 A, float2 B) const {
-    b.template store<NTXS>(on ? off : kNoRow, m * STEP * 8, A);
-    b.template store<NTXS>(on ? off : kNoRow, m * STEP * 8 + pitch8, B);
+    b.template store<NTXS>(on ? offA : kNoRow, m * STEP * 8, A);
+    b.template store<NTXS>(on ? offB : kNoRow, m * STEP * 8, B);
   }
 };
 
@@ -560,7 +564,9 @@ __global__ void __launch_bounds__((XCfg<N, XK_LR>::THREADS))
   if constexpr (lr_buf(N)) {
     const int nr = rows - rb < 2 * C::NL ? (int)(rows - rb) : 2 * C::NL;
     const int pitch8 = (int)pitch * 8;
-    const RowsBuf<C::TPT> spec{SlabBuf(S + rb * pitch, nr * pitch8), 2 * l * pitch8 + 8 * p, pitch8};
+    const bool vA = 2 * l < nr, vB = 2 * l + 1 < nr;  // an odd row count leaves a line without its second row
+    const RowsBuf<C::TPT> spec{SlabBuf(S + rb * pitch, nr * pitch8), vA ? 2 * l * pitch8 + 8 * p : kNoRow,
+                               vB ? (2 * l + 1) * pitch8 + 8 * p : kNoRow};
     merge_load<N, XK_LR>(v, line, p, spec);
     fft_line<N, C::TPT, 1, true>(v, line, p, tw);
     // the stack's loads stay behind the transform: otherwise they are issued
@@ -569,11 +575,11 @@ __global__ void __launch_bounds__((XCfg<N, XK_LR>::THREADS))
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
     const SlabBuf rw(raw + rb * N, nr * N * 4);
-    const int ro = (2 * l * N + p) * 4;
+    const int rA = vA ? (2 * l * N + p) * 4 : kNoRow, rB = vB ? ((2 * l + 1) * N + p) * 4 : kNoRow;
 #pragma unroll
     for (int m = 0; m < C::E; ++m) {
-      const float ra = rw.template load1<NTX>(ro, m * C::TPT * 4);
-      const float rc = rw.template load1<NTX>(ro, (m * C::TPT + N) * 4);
+      const float ra = rw.template load1<NTX>(rA, m * C::TPT * 4);
+      const float rc = rw.template load1<NTX>(rB, m * C::TPT * 4);
       v[m] = make_float2(lrcore(v[m].x, ra, eps), lrcore(v[m].y, rc, eps));
     }
     __syncthreads();

@@ -196,10 +196,11 @@ OtfParams OtfDev::params(const OtfTable& t, double inv_n) const {
   p.kzscale = ks[2];
   p.inv_n = (float)inv_n;
   // points with kr >= nr - 1 are zero (z filter); the bound is taken 1e-4
-  // larger, far above the rounding of kr, so it never cuts a nonzero one
+  // larger, far above the rounding of kr, so it never cuts a nonzero one.  No
+  // bound where the last ky (at most rmax / ks[1]) might not fit the kernels' int
   p.sup = kNoSupport;
   const double rmax = (t.nxotf - 1) * 1.0001;
-  if (ra && ks[0] > 0.f && ks[1] > 1e-6f && ks[0] < 1e6f && ks[1] < 1e6f)
+  if (ra && ks[0] > 0.f && ks[1] > 1e-6f && ks[0] < 1e6f && ks[1] < 1e6f && rmax / ks[1] < 1e9)
     p.sup = OtfSupport{(float)(rmax * rmax), ks[0], (float)(1.0 / ks[1])};
   return p;
 }

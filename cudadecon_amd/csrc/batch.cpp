@@ -244,7 +244,7 @@ void Batch::build_groups() {
       g.tw = ztw[kv.first];
       g.segs.ensure(sizeof(ZSeg) * kv.second.size());
       CDN_HIP(hipMemcpy(g.segs.p, kv.second.data(), sizeof(ZSeg) * kv.second.size(), hipMemcpyHostToDevice));
-      fft_prepare_ragged(g.len);
+      fft_prepare_ragged(g.len, g.buf);
       P1.zg.push_back(std::move(g));
     }
     for (const XGroup& g : P1.xg) fft_prepare_ragged(g.nx);

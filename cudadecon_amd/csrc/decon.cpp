@@ -104,8 +104,8 @@ void Fft3::setup(int x, int y, int z, hipStream_t st, DevRegion* region) {
   upload_twiddles(twx, nx, st, region);
   upload_twiddles(twy, ny, st, region);
   upload_twiddles(twz, nz, st, region);
-  fft_prepare_cols(ny, nxh, false);
-  fft_prepare_cols(nz, nxh, true);
+  fft_prepare_cols(ny, nxh, pitch, false);
+  fft_prepare_cols(nz, nxh, (long)ny * pitch, true);
 }
 
 void Fft3::col(hipStream_t st, float2* S, int axis, bool inverse, const OtfSupport& sup) const {

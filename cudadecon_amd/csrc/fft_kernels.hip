@@ -300,12 +300,27 @@ static ColRun col_run(int len, long ncols, bool narrow) {
   return r;
 }
 
-void fft_prepare_cols(int len, long ncols, bool z) {
+// the z filter's buffers (TPT planes each) take 32-bit offsets
+static bool z_buf(const CShape& cs, long line_stride) {
+  return (double)cs.TPT * (double)line_stride * 8.0 < 2147483648.0;
+}
+bool z_ragged_buf(int nz, long line_stride) { return z_buf(c_shape(nz), line_stride); }
+
+static ColRun z_run(int nz, long ncols, long line_stride) {
+  return col_run(nz, ncols, z_narrow(nz, ncols) && z_buf(c_shape(nz), line_stride));
+}
+
+void fft_prepare_cols(int len, long ncols, long line_stride, bool z) {
   FftVariant v;
-  if (fft_get_variant(len, &v) || (z ? z_narrow(len, ncols) : y_narrow(len, ncols, 1))) return;
-  if (!fft_balanced_cols(len, ncols, &v)) return;
   // compile and load (grid 0: no launch) before any stream capture
-  for (JitKernel k : {JK_COL_F, JK_COL_I, JK_Z_FILTER, JK_Z_FILTER_RA}) jit_launch(len, k, 0, 1, nullptr, nullptr, v);
+  if (!fft_get_variant(len, &v) && !(z ? z_narrow(len, ncols) : y_narrow(len, ncols, 1)) &&
+      fft_balanced_cols(len, ncols, &v))
+    for (JitKernel k : {JK_COL_F, JK_COL_I, JK_Z_FILTER, JK_Z_FILTER_RA})
+      jit_launch(len, k, 0, 1, nullptr, nullptr, v);
+  if (!z) return;
+  const ColRun run = z_run(len, ncols, line_stride);
+  if (!z_buf(run.cs, line_stride) && (run.jit || !fft_length_precompiled(len)))
+    for (JitKernel k : {JK_Z_FILTER_W, JK_Z_FILTER_RA_W}) jit_launch(len, k, 0, 1, nullptr, nullptr, run.v);
 }
 
 void launch_col_fft(int len, int inverse, hipStream_t st, float2* S, long ncols, long line_stride,
@@ -354,15 +369,9 @@ void launch_col_fft(int len, int inverse, hipStream_t st, float2* S, long ncols,
   CDN_HIP(hipGetLastError());
 }
 
-// the z filter's buffers (TPT planes each) take 32-bit offsets
-static bool z_buf(const CShape& cs, long line_stride) {
-  return (double)cs.TPT * (double)line_stride * 8.0 < 2147483648.0;
-}
-bool z_ragged_buf(int nz, long line_stride) { return z_buf(c_shape(nz), line_stride); }
-
 void launch_z_filter(int nz, hipStream_t st, float2* S, long ncols, long line_stride, long outer_stride, long ny,
                      int conj, const OtfParams& otf, const float2* tw, int nstacks, long stack_stride, bool cached) {
-  const ColRun run = col_run(nz, ncols, z_narrow(nz, ncols) && z_buf(c_shape(nz), line_stride));
+  const ColRun run = z_run(nz, ncols, line_stride);
   const CShape cs = run.cs;
   long ntiles = (ncols + cs.L - 1) / cs.L;
   if (nstacks < 1) fail("launch_z_filter: no stacks");
@@ -412,8 +421,10 @@ void launch_z_filter(int nz, hipStream_t st, float2* S, long ncols, long line_st
 long y_tile_cols(int len, long ncols) { return y_narrow(len, ncols, 0) ? kNarrowCols : c_shape(len).L; }
 long z_tile_cols(int len, long ncols) { return z_narrow(len, ncols) ? kNarrowCols : c_shape(len).L; }
 
-void fft_prepare_ragged(int len) {
+void fft_prepare_ragged(int len, bool buf) {
   if (fft_length_precompiled(len)) return;
+  if (!buf)
+    for (JitKernel k : {JK_Z_RAGGED_W, JK_Z_RAGGED_RA_W}) jit_launch(len, k, 0, 1, nullptr, nullptr);
   for (JitKernel k : {JK_X_R2C_RAGGED, JK_COL_RAGGED_F, JK_COL_RAGGED_I, JK_Z_RAGGED, JK_COL_RAGGED_FP,
                       JK_COL_RAGGED_IP, JK_Z_RAGGED_P, JK_Z_RAGGED_RA, JK_Z_RAGGED_P_RA, JK_X_C2R, JK_X_LRCORE,
                       JK_X_UPDATE})

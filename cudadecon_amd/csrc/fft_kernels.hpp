@@ -71,8 +71,8 @@ void fft_set_variant(int n, const FftVariant& v);
 // a tuned variant.
 bool fft_balanced_cols(int len, long ncols, FftVariant* v);
 // compile and load the kernels those launches will need (no GPU work); z: as
-// a z filter, else as a y transform
-void fft_prepare_cols(int len, long ncols, bool z);
+// a z filter of planes line_stride apart, else as a y transform
+void fft_prepare_cols(int len, long ncols, long line_stride, bool z);
 bool fft_get_variant(int n, FftVariant* v);
 // While one exists on this thread, every launch uses the built-in kernels of
 // its length: no tuned or single-tile variant, whose run-time compiled code
@@ -106,8 +106,9 @@ void launch_z_filter(int nz, hipStream_t st, float2* S, long ncols, long line_st
 long y_tile_cols(int len, long ncols);
 long z_tile_cols(int len, long ncols);
 // compile and load the run-time kernels the ragged launches of a length not
-// built in will use (no GPU work; call before any stream capture)
-void fft_prepare_ragged(int len);
+// built in will use (no GPU work; call before any stream capture); buf as
+// launch_z_ragged's
+void fft_prepare_ragged(int len, bool buf = true);
 void launch_col_ragged(int len, int inverse, hipStream_t st, const ColSeg* segs, int nseg, long total,
                        long cols, const float2* tw, long grid_cap = 0, bool cached = false);
 // ra: every segment's OTF is rotationally averaged (the kernel kind the

@@ -18,6 +18,7 @@
 #include <mutex>
 #include <sstream>
 #include <string>
+#include <tuple>
 #include <vector>
 
 #include "jit_sources.inc"  // kJitHeaderNames, kJitHeaderText, kJitHeaderCount (generated)
@@ -42,6 +43,14 @@ const char* const kExpr[JK_COUNT] = {"cdn::k_x_r2c<%d, false>",   "cdn::k_x_c2r<
 const char* const kOpts[] = {"--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature",
                              "-Xclang", "-packed-fp32-ops"};
 
+// Two modules per length and variant: the kernels of every stack, and those of
+// slabs too large for 32-bit offsets (JK_FIRST_WIDE on), which few programs
+// need; each is compiled when it is first asked for.
+struct Part {
+  int first, last;
+};
+constexpr Part part_of(bool wide) { return wide ? Part{JK_FIRST_WIDE, JK_COUNT} : Part{0, JK_FIRST_WIDE}; }
+
 struct Compiled {
   std::vector<char> code;
   std::string names[JK_COUNT];
@@ -52,8 +61,9 @@ struct Loaded {
 };
 
 std::mutex g_mu;
-std::map<std::pair<int, std::string>, Compiled> g_code;                 // (length, variant defines)
-std::map<std::pair<std::pair<int, int>, std::string>, Loaded> g_loaded;  // ((device, length), defines)
+using CodeKey = std::tuple<int, bool, std::string>;  // length, wide part, variant defines
+std::map<CodeKey, Compiled> g_code;
+std::map<std::pair<int, CodeKey>, Loaded> g_loaded;  // by device
 
 std::string expr(int k, int n) {
   char b[64];
@@ -84,22 +94,22 @@ std::string cache_dir() {
   return d;
 }
 
-bool load_cached(const std::string& path, Compiled& c) {
+bool load_cached(const std::string& path, Part q, Compiled& c) {
   std::ifstream f(path, std::ios::binary);
   if (!f) return false;
   std::string line;
-  for (int k = 0; k < JK_COUNT; ++k)
+  for (int k = q.first; k < q.last; ++k)
     if (!std::getline(f, c.names[k]) || c.names[k].empty()) return false;
   c.code.assign(std::istreambuf_iterator<char>(f), std::istreambuf_iterator<char>());
   return !c.code.empty();
 }
 
-void store_cached(const std::string& path, const Compiled& c) {
+void store_cached(const std::string& path, Part q, const Compiled& c) {
   const std::string tmp = path + ".tmp" + std::to_string(::getpid());
   {
     std::ofstream f(tmp, std::ios::binary);
     if (!f) return;
-    for (int k = 0; k < JK_COUNT; ++k) f << c.names[k] << '\n';
+    for (int k = q.first; k < q.last; ++k) f << c.names[k] << '\n';
     f.write(c.code.data(), (std::streamsize)c.code.size());
     if (!f) return;
   }
@@ -120,24 +130,25 @@ std::vector<std::string> split_opts(const std::string& s) {
   return out;
 }
 
-Compiled compile(int n, const std::string& defines) {
+Compiled compile(int n, bool wide, const std::string& defines) {
+  const Part q = part_of(wide);
   const std::string src = "#include \"fft_kernels_dev.hpp\"\n";
   std::string key = src + std::to_string(n) + defines;
   for (const char* o : kOpts) key += o;
-  for (const char* e : kExpr) key += e;
+  for (int k = q.first; k < q.last; ++k) key += kExpr[k];
   for (int i = 0; i < kJitHeaderCount; ++i) key += kJitHeaderText[i];
   char hex[32];
   std::snprintf(hex, sizeof hex, "%016llx", (unsigned long long)fnv1a(key));
   const std::string dir = cache_dir();
   const std::string path = dir.empty() ? "" : dir + "/fft_" + std::to_string(n) + "_" + hex + ".hsaco";
   Compiled c;
-  if (!path.empty() && load_cached(path, c)) return c;
+  if (!path.empty() && load_cached(path, q, c)) return c;
 
   hiprtcProgram prog;
   CDN_RTC(hiprtcCreateProgram(&prog, src.c_str(), "cdn_fft_jit.hip", kJitHeaderCount, kJitHeaderText,
                               kJitHeaderNames));
   std::string exprs[JK_COUNT];
-  for (int k = 0; k < JK_COUNT; ++k) {
+  for (int k = q.first; k < q.last; ++k) {
     exprs[k] = expr(k, n);
     CDN_RTC(hiprtcAddNameExpression(prog, exprs[k].c_str()));
   }
@@ -153,7 +164,7 @@ Compiled compile(int n, const std::string& defines) {
     hiprtcDestroyProgram(&prog);
     fail("run-time compilation of the FFT kernels for length " + std::to_string(n) + " failed: " + log);
   }
-  for (int k = 0; k < JK_COUNT; ++k) {
+  for (int k = q.first; k < q.last; ++k) {
     const char* lowered = nullptr;
     CDN_RTC(hiprtcGetLoweredName(prog, exprs[k].c_str(), &lowered));
     c.names[k] = lowered;
@@ -163,7 +174,7 @@ Compiled compile(int n, const std::string& defines) {
   c.code.resize(cs);
   CDN_RTC(hiprtcGetCode(prog, c.code.data()));
   hiprtcDestroyProgram(&prog);
-  if (!path.empty()) store_cached(path, c);
+  if (!path.empty()) store_cached(path, q, c);
   return c;
 }
 
@@ -188,35 +199,38 @@ std::string FftVariant::defines(int n) const {
   return d;
 }
 
-void jit_prepare(int n, const FftVariant& v) {
-  const std::string d = v.defines(n);
+static void prepare_part(const CodeKey& key) {
   {
     std::lock_guard<std::mutex> lk(g_mu);
-    if (g_code.count({n, d})) return;
+    if (g_code.count(key)) return;
   }
+  const auto& [n, wide, defines] = key;
   if (!jit_length_ok(n)) fail("FFT length " + std::to_string(n) + " is not 2,3,5,7-smooth or exceeds 16384");
   // compile outside the lock, so that several variants can compile at once
-  Compiled c = compile(n, d);
+  Compiled c = compile(n, wide, defines);
   std::lock_guard<std::mutex> lk(g_mu);
-  g_code.emplace(std::make_pair(n, d), std::move(c));
+  g_code.emplace(key, std::move(c));
 }
+
+void jit_prepare(int n, const FftVariant& v) { prepare_part(CodeKey(n, false, v.defines(n))); }
 
 void jit_launch(int n, JitKernel k, unsigned grid, unsigned block, hipStream_t st, void** args,
                 const FftVariant& v) {
-  jit_prepare(n, v);
-  const std::string d = v.defines(n);
+  const CodeKey key(n, k >= JK_FIRST_WIDE, v.defines(n));
+  prepare_part(key);
   int dev = 0;
   CDN_HIP(hipGetDevice(&dev));
   hipFunction_t fn;
   {
     std::lock_guard<std::mutex> lk(g_mu);
-    auto it = g_loaded.find({{dev, n}, d});
+    auto it = g_loaded.find({dev, key});
     if (it == g_loaded.end()) {
-      const Compiled& c = g_code.at({n, d});
+      const Compiled& c = g_code.at(key);
+      const Part q = part_of(std::get<1>(key));
       Loaded L;
       CDN_HIP(hipModuleLoadData(&L.mod, c.code.data()));
-      for (int j = 0; j < JK_COUNT; ++j) CDN_HIP(hipModuleGetFunction(&L.fn[j], L.mod, c.names[j].c_str()));
-      it = g_loaded.emplace(std::make_pair(std::make_pair(dev, n), d), L).first;
+      for (int j = q.first; j < q.last; ++j) CDN_HIP(hipModuleGetFunction(&L.fn[j], L.mod, c.names[j].c_str()));
+      it = g_loaded.emplace(std::make_pair(dev, key), L).first;
     }
     fn = it->second.fn[k];
   }

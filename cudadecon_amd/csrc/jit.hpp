@@ -27,8 +27,9 @@ enum JitKernel {
   JK_Z_FILTER_RA,
   JK_Z_RAGGED_RA,
   JK_Z_RAGGED_P_RA,
-  // _W: slabs too large for 32-bit offsets
+  // _W: slabs too large for 32-bit offsets (a module of their own)
   JK_COL_FW,
+  JK_FIRST_WIDE = JK_COL_FW,
   JK_COL_IW,
   JK_Z_FILTER_W,
   JK_Z_FILTER_RA_W,
@@ -69,9 +70,11 @@ std::string jit_cache_dir();
 
 // n is 2,3,5,7-smooth and within the lengths the kernels are sized for
 bool jit_length_ok(int n);
-// compile the kernels of length n (host only, cached); throws on failure
+// compile the kernels of length n but the _W ones (host only, cached); throws
+// on failure
 void jit_prepare(int n, const FftVariant& v = FftVariant());
-// launch kernel k of length n on the current device (loads its module once)
+// launch kernel k of length n on the current device (compiles and loads its
+// module at first need); grid 0 launches nothing
 void jit_launch(int n, JitKernel k, unsigned grid, unsigned block, hipStream_t st, void** args,
                 const FftVariant& v = FftVariant());
 

@@ -390,7 +390,8 @@ void launch_z_filter(int nz, hipStream_t st, float2* S, long ncols, long line_st
     switch (nz) {
 #define CDN_CASE(N)                                                                                             \
   case N: {                                                                                                     \
-    auto* k = ra ? k_z_filter<N, ZF_RA, true, kNarrowCols> : k_z_filter<N, ZF_ANY, true, kNarrowCols>;          \
+    auto* k = ra ? k_z_filter<N, ZF_RA, true, kNarrowCols>                                                      \
+                 : k_z_filter<N, ZF_ANY, zf_buf(N, ZF_ANY), kNarrowCols>;                                       \
     hipLaunchKernelGGL(k, dim3(grid), dim3(cs.THREADS), 0, st, S, ncols, line_stride, outer_stride, ntiles, ny, \
                        stack_stride, conj, op, tw);                                                             \
     break;                                                                                                      \
@@ -402,8 +403,8 @@ void launch_z_filter(int nz, hipStream_t st, float2* S, long ncols, long line_st
     switch (nz) {
 #define CDN_CASE(N)                                                                                             \
   case N: {                                                                                                     \
-    auto* k = ra ? (buf ? k_z_filter<N, ZF_RA, true> : k_z_filter<N, ZF_RA, false>)                             \
-                 : (buf ? k_z_filter<N, ZF_ANY, true> : k_z_filter<N, ZF_ANY, false>);                          \
+    auto* k = ra ? (buf ? k_z_filter<N, ZF_RA> : k_z_filter<N, ZF_RA, false>)                                   \
+                 : (buf ? k_z_filter<N, ZF_ANY> : k_z_filter<N, ZF_ANY, false>);                                \
     hipLaunchKernelGGL(k, dim3(grid), dim3(cs.THREADS), 0, st, S, ncols, line_stride, outer_stride, ntiles, ny, \
                        stack_stride, conj, op, tw);                                                             \
     break;                                                                                                      \
@@ -484,8 +485,9 @@ void launch_col_ragged(int len, int inverse, hipStream_t st, const ColSeg* segs,
 template <int N, int COLS>
 static auto z_ragged_n(bool pers, bool ra, bool buf) {
   if (COLS == 0 && !buf) return ra ? k_z_ragged<N, false, ZF_RA, false> : k_z_ragged<N, false, ZF_ANY, false>;
-  return pers ? (ra ? k_z_ragged<N, true, ZF_RA, true, COLS> : k_z_ragged<N, true, ZF_ANY, true, COLS>)
-              : (ra ? k_z_ragged<N, false, ZF_RA, true, COLS> : k_z_ragged<N, false, ZF_ANY, true, COLS>);
+  constexpr bool B = zf_buf(N, ZF_ANY);
+  return pers ? (ra ? k_z_ragged<N, true, ZF_RA, true, COLS> : k_z_ragged<N, true, ZF_ANY, B, COLS>)
+              : (ra ? k_z_ragged<N, false, ZF_RA, true, COLS> : k_z_ragged<N, false, ZF_ANY, B, COLS>);
 }
 
 void launch_z_ragged(int nz, hipStream_t st, const ZSeg* segs, int nseg, long total, long cols, int conj,

@@ -56,13 +56,13 @@ ZFilterKernel* cached_z_filter(int n, bool ra, bool narrow) {
   if (narrow) {
 #define CDN_CASE(N) \
   case N:           \
-    return ra ? k_z_filter<N, ZF_RA, true, kNarrowCols> : k_z_filter<N, ZF_ANY, true, kNarrowCols>;
+    return ra ? k_z_filter<N, ZF_RA, true, kNarrowCols> : k_z_filter<N, ZF_ANY, zf_buf(N, ZF_ANY), kNarrowCols>;
     CDN_PICK(CDN_NARROW_LENGTHS, CDN_CASE)
 #undef CDN_CASE
   }
 #define CDN_CASE(N) \
   case N:           \
-    return ra ? k_z_filter<N, ZF_RA, true> : k_z_filter<N, ZF_ANY, true>;
+    return ra ? k_z_filter<N, ZF_RA> : k_z_filter<N, ZF_ANY>;
   CDN_PICK(CDN_FFT_LENGTHS, CDN_CASE)
 #undef CDN_CASE
 }
@@ -86,7 +86,8 @@ ZRaggedKernel* cached_z_ragged(int n, bool ra, bool narrow) {
   if (narrow) {
 #define CDN_CASE(N) \
   case N:           \
-    return ra ? k_z_ragged<N, false, ZF_RA, true, kNarrowCols> : k_z_ragged<N, false, ZF_ANY, true, kNarrowCols>;
+    return ra ? k_z_ragged<N, false, ZF_RA, true, kNarrowCols>    \
+              : k_z_ragged<N, false, ZF_ANY, zf_buf(N, ZF_ANY), kNarrowCols>;
     CDN_PICK(CDN_NARROW_LENGTHS, CDN_CASE)
 #undef CDN_CASE
   }

@@ -920,10 +920,21 @@ template <int N, int KIND> struct ZRows {
   static constexpr int R = zf_rows(N, KIND);
 };
 
+// Whether the z filter takes its planes through buffers (SlabBuf).  The 3-D
+// kind, whose interpolation holds eight table values and needs the registers,
+// does so at 64 and 128 points only.  ms per launch, addresses -> buffers: 64
+// points 0.351 -> 0.345 (64 x 2048 x 1024), 128 0.350 -> 0.338 (128 x 1024 x 1024);
+// 256 0.193 -> 0.221 (256 x 512 x 512; 14 -> 17 registers spilled), 810 0.264 ->
+// 0.305 (810 x 192 x 256; 8 -> 29), 192 0.285 -> 0.298, 96 0.285 -> 0.291, 256 in
+// tiles of 16 columns 0.0322 -> 0.0326; 384, 512, 768, 1024 and run-time lengths
+// (48, 70, 90, 100, 600) the same within 1%.
+constexpr bool zf_buf(int N, int kind) { return kind == ZF_RA || N == 64 || N == 128; }
+
 // filter_kernel / filterConj_kernel (src/RLgpuImpl.cu:331-350) with the OTF
 // value computed on the fly as in dev_otfinterpolate (src/RLgpuImpl.cu:228-329)
-// BUF: TPT rows (planes) span less than 2^31 bytes (z_buf).
-template <int N, int KIND = ZF_ANY, bool BUF = true, int COLS = 0>
+// BUF: TPT rows (planes) span less than 2^31 bytes (z_buf) and the kind gains
+// from buffers (zf_buf).
+template <int N, int KIND = ZF_ANY, bool BUF = zf_buf(N, KIND), int COLS = 0>
 __global__ void __launch_bounds__((CCfg<N, COLS>::THREADS))
     __attribute__((amdgpu_waves_per_eu(zf_waves(N, KIND, COLS))))
     k_z_filter(float2* __restrict__ S, long ncols, long line_stride, long outer_stride, long ntiles, long ny,
@@ -945,7 +956,7 @@ __global__ void __launch_bounds__((CCfg<N, COLS>::THREADS))
 // and OTFs in one launch (ZSeg per stack); items and PERSIST as k_col_ragged.
 // KIND as k_z_filter's (ZF_RA: every segment's table is rotationally
 // averaged), so that each stack runs the code its one-stack engine runs.
-template <int N, bool PERSIST, int KIND = ZF_ANY, bool BUF = true, int COLS = 0>
+template <int N, bool PERSIST, int KIND = ZF_ANY, bool BUF = zf_buf(N, KIND), int COLS = 0>
 __global__ void __launch_bounds__((CCfg<N, COLS>::THREADS))
     __attribute__((amdgpu_waves_per_eu(zf_waves(N, KIND, COLS))))
     k_z_ragged(const ZSeg* __restrict__ segs, int nseg, long total, int conj, const float2* __restrict__ tw) {

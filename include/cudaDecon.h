@@ -243,7 +243,8 @@ int cudaDecon_device_copy(void* dst, const void* src, size_t bytes, int kind);
  *   spanning all stacks of that length whatever their other sizes (about
  *   3 nx + 4 ny + 2 nz + 2 launches per iteration for the distinct lengths);
  *   4 = the mode-3 schedule captured once into a hipGraph and replayed.
- * Every mode gives each stack bitwise the result of a one-stack engine.
+ * Every mode gives each stack bitwise the result of a one-stack engine (grouped
+ * modes with a 3-D OTF at z lengths with a factor of 5: to FP32 rounding).
  * *ms receives the device time of the whole batch.  set_raw / set_raw_block
  * reject stacks holding NaN or Inf. */
 typedef struct cudaDecon_batch cudaDecon_batch;

@@ -10,8 +10,8 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 LENGTH = 245  # used by no other test: its code is not in this process yet
-# k_col<N, inverse, false>, k_z_filter<N, kind, false>, k_z_ragged<N, persistent, kind, false>
-WIDE = re.compile(rb"k_colILi\d+ELb[01]ELb0E|k_z_filterILi\d+ELi[01]ELb0E|k_z_raggedILi\d+ELb[01]ELi[01]ELb0E")
+# k_col<N, inverse, false>, and of the averaged kind k_z_filter<N, 1, false>, k_z_ragged<N, persistent, 1, false>
+WIDE = re.compile(rb"k_colILi\d+ELb[01]ELb0E|k_z_filterILi\d+ELi1ELb0E|k_z_raggedILi\d+ELb[01]ELi1ELb0E")
 
 
 def test_preparing_a_length_leaves_out_the_wide_slab_kernels(cdn, tmp_path):

@@ -428,6 +428,8 @@ double Batch::run(int iters, int mode) {
       for (const XGroup& g : P.xg)
         if (x_update_rows_per_block(g.nx) != g.rpb) stale = true;  // the autotuner changed an x launch shape
     if (stale) build_groups();
+    for (const Partition& P : parts)
+      for (const XGroup& g : P.xg) fft_prepare_x_variant(g.nx, spec_cached(a_spec.bytes));
   }
   if (mode == BATCH_GRAPH) capture(cap_streams, iters, false);
   if (mode == BATCH_GROUPED_GRAPH) capture(cap_grouped, iters, true);

@@ -245,6 +245,7 @@ void RLEngine::setup(int nx, int ny, int nz, const OtfTable& t, const float ksca
     g.ensure(vb);
     spec.ensure(sb);
   }
+  fft_prepare_variants(nx, ny, nz, fft.nxh, fft.pitch, nstacks);
   nb_part = x_update_blocks(nx, (long)ny * nz);
   // room for any x-pass launch shape the autotuner may install later
   obtain(part, sizeof(double) * 2 * (size_t)x_update_blocks_max((long)ny * nz) * nstacks, region);
@@ -283,7 +284,10 @@ void RLEngine::bind_lambdas(DevRegion& region, int n) {
   region.give(lam, sizeof(double) * 4 * (size_t)nstacks * (size_t)std::max(n, 1));
 }
 
-void RLEngine::prepare(int n) { lam.ensure(sizeof(double) * 4 * (size_t)nstacks * (size_t)std::max(n, 1)); }
+void RLEngine::prepare(int n) {
+  lam.ensure(sizeof(double) * 4 * (size_t)nstacks * (size_t)std::max(n, 1));
+  fft_prepare_variants(fft.nx, fft.ny, fft.nz, fft.nxh, fft.pitch, nstacks);
+}
 
 std::vector<const void*> RLEngine::device_addresses() const {
   return {raw.p, xa.p, xb.p, y.p, g.p, spec.p, part.p, lam.p, otf.raw.p, otf.tz.p, otf.tz2.p,

@@ -104,6 +104,15 @@ void fft_clear_variants() {
   g_variants.clear();
 }
 
+// The tuned variant that shapes an x pass of length nx.  A variant that shapes
+// only the column passes of its length leaves the x passes their built-in
+// kernels (and their cached build).
+static bool x_variant(int nx, FftVariant* v, bool cached = false) {
+  if (!fft_get_variant(nx, v) || v->xthreads <= 0) return false;
+  v->cached = cached;
+  return true;
+}
+
 #define CDN_LAUNCH(kernel, N, grid, block, ...) \
   hipLaunchKernelGGL(kernel<N>, dim3(grid), dim3(block), 0, st, __VA_ARGS__)
 
@@ -111,7 +120,7 @@ void launch_x_r2c(int nx, hipStream_t st, const float* X, const float* Xp, float
                   float2* S, long rows, long pitch, const float2* tw, long stack_rows, const long* row_starts,
                   int nstk, bool cached) {
   FftVariant tv;
-  const bool tuned = fft_get_variant(nx, &tv);
+  const bool tuned = x_variant(nx, &tv, cached);
   const XShape xs = x_shape(nx, tuned ? tv.xthreads : -1, XK_R2C);
   const unsigned grid = grid1(((rows + 1) / 2 + xs.NL - 1) / xs.NL);
   if (stack_rows <= 0) stack_rows = rows;
@@ -147,7 +156,7 @@ void launch_x_r2c(int nx, hipStream_t st, const float* X, const float* Xp, float
 
 void launch_x_c2r(int nx, hipStream_t st, const float2* S, float* out, long rows, long pitch, const float2* tw) {
   FftVariant tv;
-  const bool tuned = fft_get_variant(nx, &tv);
+  const bool tuned = x_variant(nx, &tv);
   const XShape xs = x_shape(nx, tuned ? tv.xthreads : -1);
   const unsigned grid = grid1(((rows + 1) / 2 + xs.NL - 1) / xs.NL);
   void* args[] = {&S, &out, &rows, &pitch, &tw};
@@ -171,7 +180,7 @@ void launch_x_c2r(int nx, hipStream_t st, const float2* S, float* out, long rows
 void launch_x_lrcore(int nx, hipStream_t st, float2* S, const float* raw, long rows, long pitch, const float2* tw,
                      float eps, bool cached) {
   FftVariant tv;
-  const bool tuned = fft_get_variant(nx, &tv);
+  const bool tuned = x_variant(nx, &tv, cached);
   const XShape xs = x_shape(nx, tuned ? tv.xthreads : -1, XK_LR);
   const unsigned grid = grid1(((rows + 1) / 2 + xs.NL - 1) / xs.NL);
   void* args[] = {&S, &raw, &rows, &pitch, &tw, &eps};
@@ -196,7 +205,7 @@ void launch_x_lrcore(int nx, hipStream_t st, float2* S, const float* raw, long r
 
 int x_update_blocks(int nx, long rows) {
   FftVariant tv;
-  const bool tuned = fft_get_variant(nx, &tv);
+  const bool tuned = x_variant(nx, &tv);
   const XShape xs = x_shape(nx, tuned ? tv.xthreads : -1);
   return (int)(((rows + 1) / 2 + xs.NL - 1) / xs.NL);
 }
@@ -205,14 +214,14 @@ int x_update_blocks_max(long rows) { return (int)((rows + 1) / 2); }
 
 long x_update_rows_per_block(int nx) {
   FftVariant tv;
-  const bool tuned = fft_get_variant(nx, &tv);
+  const bool tuned = x_variant(nx, &tv);
   return 2L * x_shape(nx, tuned ? tv.xthreads : -1).NL;
 }
 
 int launch_x_update(int nx, hipStream_t st, const float2* S, const float* Y, float* Xout, float* G, double* part,
                     int dots, long rows, long pitch, const float2* tw, bool cached) {
   FftVariant tv;
-  const bool tuned = fft_get_variant(nx, &tv);
+  const bool tuned = x_variant(nx, &tv, cached);
   const XShape xs = x_shape(nx, tuned ? tv.xthreads : -1);
   const int nb = (int)(((rows + 1) / 2 + xs.NL - 1) / xs.NL);
   void* args[] = {&S, &Y, &Xout, &G, &part, &dots, &rows, &pitch, &tw};
@@ -285,16 +294,31 @@ static bool z_narrow(int len, long ncols) {
 }
 
 // How a column pass runs: the tuned variant of the length, else narrow tiles,
-// else one tile of all columns, else the length's own shape.
+// else one tile of all columns, else the length's own shape.  A variant that
+// leaves the tile's shape alone (loads, renumbering, OTF rows) runs narrow
+// tiles where the built-in kernels do, and every tuned variant the build that
+// keeps the spectrum in cache where they do.
 struct ColRun {
   CShape cs;
   bool jit, narrow;
   FftVariant v;
 };
-static ColRun col_run(int len, long ncols, bool narrow) {
+static FftVariant col_flavour(FftVariant v, int len, bool narrow, bool cached) {
+  if (narrow && v.cols == 0 && v.col_tpt == 0) {
+    v.cols = kNarrowCols;
+    if (c_shape(len, kNarrowCols).TPT != c_shape(len).TPT) v.col_tpt = c_shape(len, kNarrowCols).TPT;
+  }
+  v.cached = cached;
+  return v;
+}
+static ColRun col_run(int len, long ncols, bool narrow, bool cached) {
   ColRun r{};
-  r.jit = fft_get_variant(len, &r.v);
+  r.jit = fft_get_variant(len, &r.v) && r.v.shapes_cols();
   r.narrow = !r.jit && narrow;
+  if (r.jit)
+    r.v = col_flavour(r.v, len, narrow, cached);
+  else
+    r.v = FftVariant();
   if (!r.jit && !r.narrow) r.jit = fft_balanced_cols(len, ncols, &r.v);
   r.cs = r.narrow ? c_shape(len, kNarrowCols) : c_shape(len, r.jit ? r.v.cols : -1, r.jit ? r.v.col_tpt : -1);
   return r;
@@ -306,29 +330,62 @@ static bool z_buf(const CShape& cs, long line_stride) {
 }
 bool z_ragged_buf(int nz, long line_stride) { return z_buf(c_shape(nz), line_stride); }
 
-static ColRun z_run(int nz, long ncols, long line_stride) {
-  return col_run(nz, ncols, z_narrow(nz, ncols) && z_buf(c_shape(nz), line_stride));
+static bool z_runs_narrow(int nz, long ncols, long line_stride) {
+  return z_narrow(nz, ncols) && z_buf(c_shape(nz), line_stride);
+}
+static ColRun z_run(int nz, long ncols, long line_stride, bool cached) {
+  return col_run(nz, ncols, z_runs_narrow(nz, ncols, line_stride), cached);
+}
+// a slab's rows by 32-bit offsets (always the case for y transforms: at most
+// 16384 rows of 8208 columns)
+static bool col_buf32(int len, long line_stride) { return (double)len * (double)line_stride * 8.0 < 2147483648.0; }
+static bool col_runs_narrow(int len, long ncols, long line_stride, long n_outer) {
+  return col_buf32(len, line_stride) && y_narrow(len, ncols, n_outer);
 }
 
 void fft_prepare_cols(int len, long ncols, long line_stride, bool z) {
   FftVariant v;
   // compile and load (grid 0: no launch) before any stream capture
-  if (!fft_get_variant(len, &v) && !(z ? z_narrow(len, ncols) : y_narrow(len, ncols, 1)) &&
+  if (!(fft_get_variant(len, &v) && v.shapes_cols()) && !(z ? z_narrow(len, ncols) : y_narrow(len, ncols, 1)) &&
       fft_balanced_cols(len, ncols, &v))
     for (JitKernel k : {JK_COL_F, JK_COL_I, JK_Z_FILTER, JK_Z_FILTER_RA})
       jit_launch(len, k, 0, 1, nullptr, nullptr, v);
   if (!z) return;
-  const ColRun run = z_run(len, ncols, line_stride);
+  const ColRun run = z_run(len, ncols, line_stride, false);
   if (!z_buf(run.cs, line_stride) && (run.jit || !fft_length_precompiled(len)))
     for (JitKernel k : {JK_Z_FILTER_W, JK_Z_FILTER_RA_W}) jit_launch(len, k, 0, 1, nullptr, nullptr, run.v);
 }
 
+GridFlavours grid_flavours(int nx, int ny, int nz, long nxh, long pitch, int nstacks) {
+  GridFlavours f;
+  f.cached = spec_cached(sizeof(float2) * (size_t)pitch * ny * nz * nstacks);
+  f.y_narrow = col_runs_narrow(ny, nxh, pitch, (long)nz * nstacks);
+  f.z_narrow = z_runs_narrow(nz, nxh, (long)ny * pitch);
+  return f;
+}
+FftVariant fft_column_flavour(int len, const FftVariant& v, bool narrow, bool cached) {
+  return col_flavour(v, len, narrow, cached);
+}
+
+void fft_prepare_variants(int nx, int ny, int nz, long nxh, long pitch, int nstacks) {
+  FftVariant v;
+  const bool any_x = x_variant(nx, &v);
+  const bool any_y = fft_get_variant(ny, &v) && v.shapes_cols(), any_z = fft_get_variant(nz, &v) && v.shapes_cols();
+  if (!any_x && !any_y && !any_z) return;
+  const GridFlavours f = grid_flavours(nx, ny, nz, nxh, pitch, nstacks);
+  if (any_x && x_variant(nx, &v, f.cached)) jit_launch(nx, JK_X_R2C, 0, 1, nullptr, nullptr, v);
+  if (any_y) jit_launch(ny, JK_COL_F, 0, 1, nullptr, nullptr, col_run(ny, nxh, f.y_narrow, f.cached).v);
+  if (any_z) jit_launch(nz, JK_Z_FILTER, 0, 1, nullptr, nullptr, col_run(nz, nxh, f.z_narrow, f.cached).v);
+}
+void fft_prepare_x_variant(int nx, bool cached) {
+  FftVariant v;
+  if (x_variant(nx, &v, cached)) jit_launch(nx, JK_X_R2C, 0, 1, nullptr, nullptr, v);
+}
+
 void launch_col_fft(int len, int inverse, hipStream_t st, float2* S, long ncols, long line_stride,
                     long outer_stride, long n_outer, const float2* tw, const OtfSupport& sup, bool cached) {
-  // a slab's rows by 32-bit offsets (always the case for y transforms: at
-  // most 16384 rows of 8208 columns)
-  const bool buf = (double)len * (double)line_stride * 8.0 < 2147483648.0;
-  const ColRun run = col_run(len, ncols, buf && y_narrow(len, ncols, n_outer));
+  const bool buf = col_buf32(len, line_stride);
+  const ColRun run = col_run(len, ncols, col_runs_narrow(len, ncols, line_stride, n_outer), cached);
   const CShape cs = run.cs;
   long ntiles = (ncols + cs.L - 1) / cs.L;
   const unsigned grid = grid1(ntiles * n_outer);
@@ -371,7 +428,7 @@ void launch_col_fft(int len, int inverse, hipStream_t st, float2* S, long ncols,
 
 void launch_z_filter(int nz, hipStream_t st, float2* S, long ncols, long line_stride, long outer_stride, long ny,
                      int conj, const OtfParams& otf, const float2* tw, int nstacks, long stack_stride, bool cached) {
-  const ColRun run = z_run(nz, ncols, line_stride);
+  const ColRun run = z_run(nz, ncols, line_stride, cached);
   const CShape cs = run.cs;
   long ntiles = (ncols + cs.L - 1) / cs.L;
   if (nstacks < 1) fail("launch_z_filter: no stacks");

@@ -28,7 +28,7 @@ void fft_twiddles(int n, float2* out);
 // Whether an iteration's passes should keep a spectrum of `bytes` in the
 // memory-side cache (256 MB): `cached` of the launchers below, which then run
 // the kernels that access it with cached instructions (real volumes stream as
-// before; lengths without built-in kernels and tuned shapes ignore it).  Each
+// before; lengths without built-in kernels ignore it unless tuned).  Each
 // pass then finds the spectrum where the one before left it.  ms per iteration,
 // streaming -> cached: 64 x 512 x 512 (69 MB) 0.329 -> 0.306, 128 x 512 x 512
 // (138 MB) 0.567 -> 0.517, 64 x 768 x 768 (151 MB) 0.687 -> 0.595, 192 x 512 x 512
@@ -74,6 +74,18 @@ bool fft_balanced_cols(int len, long ncols, FftVariant* v);
 // a z filter of planes line_stride apart, else as a y transform
 void fft_prepare_cols(int len, long ncols, long line_stride, bool z);
 bool fft_get_variant(int n, FftVariant* v);
+// What the passes of a grid run: the spectrum kept in cache, tiles of 16
+// columns in the y passes and in the z filter.
+struct GridFlavours {
+  bool cached = false, y_narrow = false, z_narrow = false;
+};
+GridFlavours grid_flavours(int nx, int ny, int nz, long nxh, long pitch, int nstacks = 1);
+// a column variant as a launch of such a grid compiles it
+FftVariant fft_column_flavour(int len, const FftVariant& v, bool narrow, bool cached);
+// compile and load what the tuned variants of a grid's lengths will launch (no
+// GPU work; before any stream capture); x: of one x length
+void fft_prepare_variants(int nx, int ny, int nz, long nxh, long pitch, int nstacks);
+void fft_prepare_x_variant(int nx, bool cached);
 // While one exists on this thread, every launch uses the built-in kernels of
 // its length: no tuned or single-tile variant, whose run-time compiled code
 // would have to be loaded (column results are bitwise the same).

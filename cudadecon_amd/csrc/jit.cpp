@@ -196,6 +196,7 @@ std::string FftVariant::defines(int n) const {
   if (col_tpt > 0) d += " -DCDN_CTPT_OVERRIDE=" + std::to_string(n) + "," + std::to_string(col_tpt);
   if (zf_waves > 0) d += " -DCDN_ZF_WAVES=" + std::to_string(zf_waves);
   if (zf_rows != 0) d += " -DCDN_ZF_ROWS_OVERRIDE=" + std::to_string(n) + "," + std::to_string(zf_rows);
+  if (cached) d += " -DCDN_SPEC_CACHED=1";
   return d;
 }
 

@@ -53,9 +53,16 @@ struct FftVariant {
   int col_tpt = 0;
   int zf_waves = 0;
   int zf_rows = 0;
+  // not a choice: the launch keeps its spectrum in cache (spec_cached), set by
+  // the launchers
+  bool cached = false;
   bool is_default() const {
     return cols == 0 && xthreads == 0 && col_nt_load < 0 && xcd_remap < 0 && col_tpt == 0 && zf_waves == 0 &&
            zf_rows == 0;
+  }
+  // whether it shapes the column passes (the x passes: xthreads > 0)
+  bool shapes_cols() const {
+    return cols > 0 || col_nt_load >= 0 || xcd_remap >= 0 || col_tpt > 0 || zf_waves > 0 || zf_rows != 0;
   }
   // -D options that build this variant for length n
   std::string defines(int n) const;

@@ -19,7 +19,12 @@
 // results are bitwise those of the defaults; an x-pass variant also regroups
 // the dot products' per-block partial sums (FP64, another summation order).  Candidates are compiled at run time (hipRTC),
 // several at once; decisions are cached in <cache>/tune_gfx950_v2.txt keyed
-// by length, role and the grid timed.
+// by length, role and the grid timed.  The roles carry what the grid's passes
+// run beside their shapes: c a spectrum kept in cache, n tiles of 16 columns
+// (decisions without them were timed on kernels that such grids no longer run).
+// Every candidate is timed as the grid would launch it, the built-in kernels
+// among them: with the OTF's support bound, in the cached build where the
+// spectrum fits it.
 #include "tune.hpp"
 
 #include "common.hpp"
@@ -36,6 +41,7 @@
 #include <fstream>
 #include <map>
 #include <memory>
+#include <set>
 #include <sstream>
 #include <thread>
 
@@ -105,17 +111,21 @@ struct Bench {
   OtfDev D;
   DevBuf vol, spec, aux, part;
   hipStream_t st = nullptr;
+  bool cached = false;
+  OtfParams op{};
   void setup(const std::array<int, 3>& g, hipStream_t s) {
     st = s;
     F.setup(g[2], g[1], g[0], st);
-    // a rotationally averaged table of 33 radii x 17 kz samples, scaled so
-    // that its support ends at 70% of the x and y Nyquist frequencies: the
-    // z filter interpolates in about 40% of the columns, as with a real OTF
+    cached = grid_flavours(F.nx, F.ny, F.nz, F.nxh, F.pitch).cached;
+    // a rotationally averaged table of 33 radii x 17 kz samples that ends at
+    // the x and y Nyquist frequencies, as with a PSF sampled like the data: the
+    // y passes and the z filter move 79% of the columns
     const int nr = 33, nzo = 17;
     const std::vector<float> tab((size_t)2 * nzo * nr, 0.5f);
     T.set_from_image(tab.data(), 2 * nzo, nr, 1, 1.f, 1.f);
-    const float ks[3] = {(nr - 1) / (0.35f * g[2]), (nr - 1) / (0.35f * g[1]), (nzo - 1) / (0.35f * g[0])};
+    const float ks[3] = {(nr - 1) / (0.5f * g[2]), (nr - 1) / (0.5f * g[1]), (nzo - 1) / (0.5f * g[0])};
     D.setup(T, ks, g[0], st);
+    op = D.params(T, 1.0 / (double)F.nvox);
     vol.ensure(sizeof(float) * F.nvox);
     aux.ensure(sizeof(float) * F.nvox);
     spec.ensure(sizeof(float2) * F.nspec);
@@ -129,16 +139,17 @@ struct Bench {
     float2* S = spec.as<float2>();
     if (role == 0) {
       launch_x_r2c(F.nx, st, vol.as<float>(), nullptr, nullptr, nullptr, XIN_PLAIN, S, rows, F.pitch,
-                   F.twx.as<float2>());
-      launch_x_lrcore(F.nx, st, S, vol.as<float>(), rows, F.pitch, F.twx.as<float2>(), FLT_EPSILON);
+                   F.twx.as<float2>(), 0, nullptr, 0, cached);
+      launch_x_lrcore(F.nx, st, S, vol.as<float>(), rows, F.pitch, F.twx.as<float2>(), FLT_EPSILON, cached);
       launch_x_update(F.nx, st, S, vol.as<float>(), aux.as<float>(), aux.as<float>(), part.as<double>(), 1, rows,
-                      F.pitch, F.twx.as<float2>());
+                      F.pitch, F.twx.as<float2>(), cached);
     } else if (role == 1) {
-      F.col(st, S, 1, false);
-      F.col(st, S, 1, true);
+      for (int inverse : {0, 1})
+        launch_col_fft(F.ny, inverse, st, S, F.nxh, F.pitch, (long)F.ny * F.pitch, F.nz, F.twy.as<float2>(), op.sup,
+                       cached);
     } else {
-      launch_z_filter(F.nz, st, S, F.nxh, (long)F.ny * F.pitch, F.pitch, F.ny, 0, D.params(T, 1.0 / F.nvox),
-                      F.twz.as<float2>());
+      launch_z_filter(F.nz, st, S, F.nxh, (long)F.ny * F.pitch, F.pitch, F.ny, 0, op, F.twz.as<float2>(), 1, 0,
+                      cached);
     }
   }
 };
@@ -173,7 +184,30 @@ std::string vstr(const FftVariant& v) {
   return o.str();
 }
 
-std::string gkey(int n, const char* role, const std::array<int, 3>& g) {
+GridFlavours flavours(const std::array<int, 3>& g) {
+  return grid_flavours(g[2], g[1], g[0], g[2] / 2 + 1, Fft3::pitch_of(g[2]));
+}
+
+// what a length's column candidates are compiled as: for the y passes of one
+// grid and for the z filter of another
+std::vector<FftVariant> col_flavours(int n, const Roles& r, const FftVariant& v) {
+  std::vector<FftVariant> out;
+  if (v.is_default()) return out;
+  if (r.y) out.push_back(fft_column_flavour(n, v, flavours(r.gy).y_narrow, flavours(r.gy).cached));
+  if (r.z) out.push_back(fft_column_flavour(n, v, flavours(r.gz).z_narrow, flavours(r.gz).cached));
+  return out;
+}
+
+std::string x_role(const Roles& r) { return flavours(r.gx).cached ? "xc" : "x"; }
+std::string col_role(const Roles& r) {
+  std::string s = r.y && r.z ? "yz" : (r.y ? "y" : "z");
+  const GridFlavours fy = r.y ? flavours(r.gy) : GridFlavours(), fz = r.z ? flavours(r.gz) : GridFlavours();
+  if (fy.cached || fz.cached) s += "c";
+  if (fy.y_narrow || fz.z_narrow) s += "n";
+  return s;
+}
+
+std::string gkey(int n, const std::string& role, const std::array<int, 3>& g) {
   std::ostringstream o;
   o << n << ' ' << role << ' ' << g[0] << 'x' << g[1] << 'x' << g[2];
   return o.str();
@@ -205,8 +239,11 @@ void append_cache(const std::string& path, const std::string& key, const FftVari
 // compile (hipRTC, on several threads) every variant that is not built in
 void prepare_parallel(const std::vector<std::pair<int, FftVariant>>& todo) {
   std::vector<std::pair<int, FftVariant>> jit;
+  std::set<std::pair<int, std::string>> seen;
   for (auto& t : todo)
-    if (!t.second.is_default() || !fft_length_precompiled(t.first)) jit.push_back(t);
+    if ((!t.second.is_default() || !fft_length_precompiled(t.first)) &&
+        seen.emplace(t.first, t.second.defines(t.first)).second)
+      jit.push_back(t);
   const unsigned nth = std::max(1u, std::min(8u, std::thread::hardware_concurrency()));
   std::vector<std::thread> pool;
   std::vector<std::string> errs(nth);
@@ -251,9 +288,13 @@ std::string autotune(const std::vector<std::array<int, 3>>& grids, int reps, boo
   std::vector<std::pair<int, FftVariant>> todo;
   for (auto& [n, r] : lengths) {
     if (r.x)
-      for (const FftVariant& v : x_candidates(n)) todo.push_back({n, v});
+      for (FftVariant v : x_candidates(n)) {
+        v.cached = !v.is_default() && flavours(r.gx).cached;
+        todo.push_back({n, v});
+      }
     if (r.y || r.z)
-      for (const FftVariant& v : col_candidates(n)) todo.push_back({n, v});
+      for (const FftVariant& v : col_candidates(n))
+        for (const FftVariant& w : col_flavours(n, r, v)) todo.push_back({n, w});
   }
   prepare_parallel(todo);
 
@@ -278,7 +319,7 @@ std::string autotune(const std::vector<std::array<int, 3>>& grids, int reps, boo
       rep << (first ? "" : ", ") << "{\"n\": " << n;
       first = false;
       if (r.x) {
-        const std::string key = gkey(n, "x", r.gx);
+        const std::string key = gkey(n, x_role(r), r.gx);
         FftVariant bx;
         if (cache.count(key)) {
           bx = cache[key];
@@ -303,7 +344,7 @@ std::string autotune(const std::vector<std::array<int, 3>>& grids, int reps, boo
         best.xthreads = bx.xthreads;
       }
       if (r.y || r.z) {
-        const std::string key = gkey(n, r.y && r.z ? "yz" : (r.y ? "y" : "z"), r.y ? r.gy : r.gz);
+        const std::string key = gkey(n, col_role(r), r.y ? r.gy : r.gz);
         FftVariant bc;
         if (cache.count(key)) {
           bc = cache[key];
@@ -345,7 +386,10 @@ std::string autotune(const std::vector<std::array<int, 3>>& grids, int reps, boo
                 w.zf_rows = rows;
                 zc.push_back({n, w});
               }
-            prepare_parallel(zc);
+            std::vector<std::pair<int, FftVariant>> zf;
+            for (auto& [len, w] : zc)
+              zf.push_back({len, fft_column_flavour(len, w, flavours(r.gz).z_narrow, flavours(r.gz).cached)});
+            prepare_parallel(zf);
             fft_set_variant(n, bc);
             double tb = time_role(bench(r.gz), 2, reps);
             rep << ", \"z_filter\": [[" << vstr(bc) << ", " << tb << "]";
@@ -373,7 +417,19 @@ std::string autotune(const std::vector<std::array<int, 3>>& grids, int reps, boo
         best.zf_rows = bc.zf_rows;
       }
       fft_set_variant(n, best);
-      if (!best.is_default()) jit_prepare(n, best);
+      std::vector<std::pair<int, FftVariant>> used;
+      if (r.x && best.xthreads > 0) {
+        FftVariant v = best;
+        v.cached = flavours(r.gx).cached;
+        used.push_back({n, v});
+      }
+      if (best.shapes_cols())
+        for (const FftVariant& v : col_flavours(n, r, best)) used.push_back({n, v});
+      for (size_t i = 0, m = used.size(); i < m; ++i) {  // and the streaming build, for single transforms
+        used.push_back(used[i]);
+        used.back().second.cached = false;
+      }
+      prepare_parallel(used);
       rep << ", \"chosen\": " << vstr(best) << "}";
     }
     benches.clear();

@@ -79,10 +79,13 @@ namespace {
 std::mutex g_vmu;
 std::map<int, FftVariant> g_variants;
 thread_local int t_builtin_only = 0;  // > 0: no run-time compiled variant
+thread_local int t_wide = 0;          // > 0: 64-bit addresses
 }  // namespace
 
 BuiltinShapesOnly::BuiltinShapesOnly() { ++t_builtin_only; }
 BuiltinShapesOnly::~BuiltinShapesOnly() { --t_builtin_only; }
+WideAddresses::WideAddresses() { ++t_wide; }
+WideAddresses::~WideAddresses() { --t_wide; }
 
 void fft_set_variant(int n, const FftVariant& v) {
   std::lock_guard<std::mutex> lk(g_vmu);
@@ -326,7 +329,7 @@ static ColRun col_run(int len, long ncols, bool narrow, bool cached) {
 
 // the z filter's buffers (TPT planes each) take 32-bit offsets
 static bool z_buf(const CShape& cs, long line_stride) {
-  return (double)cs.TPT * (double)line_stride * 8.0 < 2147483648.0;
+  return t_wide == 0 && (double)cs.TPT * (double)line_stride * 8.0 < 2147483648.0;
 }
 bool z_ragged_buf(int nz, long line_stride) { return z_buf(c_shape(nz), line_stride); }
 
@@ -384,8 +387,8 @@ void fft_prepare_x_variant(int nx, bool cached) {
 
 void launch_col_fft(int len, int inverse, hipStream_t st, float2* S, long ncols, long line_stride,
                     long outer_stride, long n_outer, const float2* tw, const OtfSupport& sup, bool cached) {
-  const bool buf = col_buf32(len, line_stride);
-  const ColRun run = col_run(len, ncols, col_runs_narrow(len, ncols, line_stride, n_outer), cached);
+  const bool buf = col_buf32(len, line_stride) && !(t_wide > 0 && sup.r2 < 0.f);
+  const ColRun run = col_run(len, ncols, buf && col_runs_narrow(len, ncols, line_stride, n_outer), cached);
   const CShape cs = run.cs;
   long ntiles = (ncols + cs.L - 1) / cs.L;
   const unsigned grid = grid1(ntiles * n_outer);

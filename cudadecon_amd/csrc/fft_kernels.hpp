@@ -94,6 +94,14 @@ struct BuiltinShapesOnly {
   ~BuiltinShapesOnly();
 };
 void fft_clear_variants();
+// While one exists on this thread, launches take the kernels with 64-bit
+// addresses whatever the stack's size (a pass with a support bound keeps its
+// buffers): the tests compare both on small stacks.
+struct WideAddresses {
+  WideAddresses();
+  ~WideAddresses();
+  WideAddresses(const WideAddresses&) = delete;
+};
 
 // a bound that no column exceeds
 constexpr OtfSupport kNoSupport{-1.f, 0.f, 0.f};

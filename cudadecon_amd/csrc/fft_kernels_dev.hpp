@@ -283,10 +283,10 @@ template <int N, int COLS = 0> struct CCfg {
 // this form 0.357).  Registers of the y transforms: 64 to 2048 points 60-92
 // -> 56-81, of the z filters 92-142 -> 84-126 at 64 to 192 points.
 // The range check is the vector offset's alone: the scalar offset is defined as
-// taking no part in it (and where it did, subtracting it from a length that it
-// exceeds would not help).  So an element past the end must be past it by its
-// vector offset, or have kNoRow there; its load returns zero, its store does
-// nothing.  Scalar offsets stay inside what the vector offset leaves.
+// taking no part in it (and where it did, a length less a larger scalar offset
+// would be no bound).  So whatever must not be touched has kNoRow, the largest
+// offset there is, as its vector offset: its load returns zero, its store does
+// nothing.
 constexpr int kNoRow = -1;  // past every end
 typedef unsigned u2v __attribute__((ext_vector_type(2)));
 struct SlabBuf {
@@ -337,14 +337,17 @@ template <int STEP> struct RowsPtr {
 };
 template <int STEP> struct RowsBuf {
   SlabBuf b;
-  int offA, offB;  // bytes: of element p of the two rows, kNoRow for a row past the last
+  // bytes: of element p of the first row, for each row (kNoRow for one past the
+  // last: the second row's distance, the pitch, stays in the scalar offset, so
+  // the choice must not be left to the range check)
+  int offA, offB, pitch8;
   __device__ __forceinline__ void load(int m, bool on, float2& A, float2& B) const {
     A = b.template load<NTXS>(on ? offA : kNoRow, m * STEP * 8);
-    B = b.template load<NTXS>(on ? offB : kNoRow, m * STEP * 8);
+    B = b.template load<NTXS>(on ? offB : kNoRow, m * STEP * 8 + pitch8);
   }
   __device__ __forceinline__ void store(int m, bool on, float2 A, float2 B) const {
     b.template store<NTXS>(on ? offA : kNoRow, m * STEP * 8, A);
-    b.template store<NTXS>(on ? offB : kNoRow, m * STEP * 8, B);
+    b.template store<NTXS>(on ? offB : kNoRow, m * STEP * 8 + pitch8, B);
   }
 };
 
@@ -542,9 +545,10 @@ __device__ __forceinline__ float lrcore(float c, float raw, float eps) {
 
 // LRcore lines that merge and split through LDS (up to 16 elements per thread
 // without a register-resident plan, and 2048 points) take their rows through
-// buffers: fewer registers (2048 points 125 -> 83, 810 points 78 -> 70), ms:
-// 1.104 -> 0.936 at 96 x 2048 x 2048, 0.161 -> 0.148 at 128 x 512 x 810,
-// 0.126 -> 0.118 for 48 stacks of 64 x 128 x 128.  Lines split by shuffles keep
+// buffers: fewer registers (2048 points 125 -> 89, 810 points 78 -> 71), ms:
+// 1.102 -> 0.910 at 96 x 2048 x 2048, 0.161 -> 0.147 at 128 x 512 x 810,
+// 0.125 -> 0.116 for 48 stacks of 64 x 128 x 128, 0.060 -> 0.054 at
+// 192 x 512 x 192 (0.066 with a vector offset per row that includes its distance).  Lines split by shuffles keep
 // addresses: 512 and 1024 points measured the same both ways (0.083; 0.593
 // against 0.597), 384 and 768 slower (0.142 -> 0.149, 0.124 -> 0.132), and the
 // R2C and update passes slower by 2% at 1024 points.
@@ -565,8 +569,8 @@ __global__ void __launch_bounds__((XCfg<N, XK_LR>::THREADS))
     const int nr = rows - rb < 2 * C::NL ? (int)(rows - rb) : 2 * C::NL;
     const int pitch8 = (int)pitch * 8;
     const bool vA = 2 * l < nr, vB = 2 * l + 1 < nr;  // an odd row count leaves a line without its second row
-    const RowsBuf<C::TPT> spec{SlabBuf(S + rb * pitch, nr * pitch8), vA ? 2 * l * pitch8 + 8 * p : kNoRow,
-                               vB ? (2 * l + 1) * pitch8 + 8 * p : kNoRow};
+    const int so = 2 * l * pitch8 + 8 * p;
+    const RowsBuf<C::TPT> spec{SlabBuf(S + rb * pitch, nr * pitch8), vA ? so : kNoRow, vB ? so : kNoRow, pitch8};
     merge_load<N, XK_LR>(v, line, p, spec);
     fft_line<N, C::TPT, 1, true>(v, line, p, tw);
     // the stack's loads stay behind the transform: otherwise they are issued
@@ -575,11 +579,11 @@ __global__ void __launch_bounds__((XCfg<N, XK_LR>::THREADS))
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
     const SlabBuf rw(raw + rb * N, nr * N * 4);
-    const int rA = vA ? (2 * l * N + p) * 4 : kNoRow, rB = vB ? ((2 * l + 1) * N + p) * 4 : kNoRow;
+    const int ro = (2 * l * N + p) * 4, rA = vA ? ro : kNoRow, rB = vB ? ro : kNoRow;
 #pragma unroll
     for (int m = 0; m < C::E; ++m) {
       const float ra = rw.template load1<NTX>(rA, m * C::TPT * 4);
-      const float rc = rw.template load1<NTX>(rB, m * C::TPT * 4);
+      const float rc = rw.template load1<NTX>(rB, (m * C::TPT + N) * 4);
       v[m] = make_float2(lrcore(v[m].x, ra, eps), lrcore(v[m].y, rc, eps));
     }
     __syncthreads();

@@ -356,7 +356,7 @@ int Deskew_interface(const float* const raw_data, int nx, int ny, int nz, float 
       dout.ensure(sizeof(float) * (size_t)xdim * ny * nz);
       copy_to_device(st, din.p, raw_data, sizeof(float) * (size_t)nx * ny * nz);
       deskew(st, din.as<float>(), nx, ny, nz, factor, dout.as<float>(), (int)xdim, extraShift, padVal);
-      copy_to_host(st, result, dout.p, sizeof(float) * (size_t)xdim * ny * nz);
+      copy_to_host(st, result, dout.p, sizeof(float) * (size_t)xdim * ny * nz, true);
     } catch (...) {
       (void)hipStreamDestroy(st);
       throw;
@@ -378,7 +378,7 @@ static int affine_common(const float* raw_data, int nx, int ny, int nz, float* r
       dout.ensure(sizeof(float) * n);
       copy_to_device(st, din.p, raw_data, sizeof(float) * n);
       affine(st, din.as<float>(), nx, ny, nz, dout.as<float>(), affMat, ra, dx, dy, dz);
-      copy_to_host(st, result, dout.p, sizeof(float) * n);
+      copy_to_host(st, result, dout.p, sizeof(float) * n, true);
     } catch (...) {
       (void)hipStreamDestroy(st);
       throw;
@@ -502,7 +502,7 @@ int cudaDecon_fft_c2r(const float* in, int nx, int ny, int nz, float* out) {
       CDN_HIP(hipMemcpy2DAsync(ds.p, sizeof(float2) * F.pitch, in, sizeof(float2) * F.nxh, sizeof(float2) * F.nxh,
                                (size_t)ny * nz, hipMemcpyHostToDevice, st));
       F.c2r(st, ds.as<float2>(), dv.as<float>());
-      copy_to_host(st, out, dv.p, sizeof(float) * F.nvox);
+      copy_to_host(st, out, dv.p, sizeof(float) * F.nvox, true);
     } catch (...) {
       (void)hipStreamDestroy(st);
       throw;
@@ -536,7 +536,7 @@ int cudaDecon_filter(float* vol, int nx, int ny, int nz, const float* otf, int o
       launch_z_filter(nz, st, S, F.nxh, (long)ny * F.pitch, F.pitch, ny, conj, op, F.twz.as<float2>());
       F.col(st, S, 1, true, op.sup);
       launch_x_c2r(nx, st, S, dv.as<float>(), (long)ny * nz, F.pitch, F.twx.as<float2>());
-      copy_to_host(st, vol, dv.p, sizeof(float) * F.nvox);
+      copy_to_host(st, vol, dv.p, sizeof(float) * F.nvox, true);
     } catch (...) {
       (void)hipStreamDestroy(st);
       throw;
@@ -577,7 +577,7 @@ int cudaDecon_wiener(float* vol, int nx, int ny, int nz, const float* otf, int o
       F.col(st, S, 2, true);
       F.col(st, S, 1, true);
       launch_x_c2r(nx, st, S, dv.as<float>(), (long)ny * nz, F.pitch, F.twx.as<float2>());
-      copy_to_host(st, vol, dv.p, sizeof(float) * F.nvox);
+      copy_to_host(st, vol, dv.p, sizeof(float) * F.nvox, true);
     } catch (...) {
       (void)hipStreamDestroy(st);
       throw;

@@ -26,6 +26,10 @@ constexpr int kMaxBufs = 4;
 // smaller copies go straight through the runtime: its pageable uploads reach
 // 33 GB/s from 4 MB on, its downloads 4 to 11
 constexpr size_t kDirectUp = 16UL << 20, kDirectDown = 2UL << 20;
+// a stream made for the call takes 50 us more for its first copies into pinned
+// memory: affine and deskew, ms through the runtime and staged: 2.1 MB 0.367 and
+// 0.420, 3 MB 0.43 and 0.465, 3.9 MB 0.505 and 0.515, 4.9 MB 0.58 and 0.54
+constexpr size_t kDirectFresh = 9UL << 19;
 // Downloads below this size keep out of each other's way: they hold the buffers
 // for the copy alone, not while their stream's kernels run, at most two wait for
 // one of them, and any more, or any beside a larger copy, go through the runtime.
@@ -145,8 +149,8 @@ void copy_to_device(hipStream_t st, void* dev, const void* host, size_t bytes) {
   }
 }
 
-void copy_to_host(hipStream_t st, void* host, const void* dev, size_t bytes) {
-  if (bytes < kDirectDown) {
+void copy_to_host(hipStream_t st, void* host, const void* dev, size_t bytes, bool fresh_stream) {
+  if (bytes < (fresh_stream ? kDirectFresh : kDirectDown)) {
     CDN_HIP(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, st));
     CDN_HIP(hipStreamSynchronize(st));
     return;

@@ -18,7 +18,7 @@ namespace cdn {
 void copy_to_device(hipStream_t st, void* dev, const void* host, size_t bytes);
 
 // device -> host, after the work already queued on `st`.  Returns once the
-// data is in the host buffer.
-void copy_to_host(hipStream_t st, void* host, const void* dev, size_t bytes);
+// data is in the host buffer.  fresh_stream: `st` was made for this call.
+void copy_to_host(hipStream_t st, void* host, const void* dev, size_t bytes, bool fresh_stream = false);
 
 }  // namespace cdn

@@ -32,10 +32,15 @@ void fft_twiddles(int n, float2* out);
 // pass then finds the spectrum where the one before left it.  ms per iteration,
 // streaming -> cached: 64 x 512 x 512 (69 MB) 0.329 -> 0.306, 128 x 512 x 512
 // (138 MB) 0.567 -> 0.517, 64 x 768 x 768 (151 MB) 0.687 -> 0.595, 192 x 512 x 512
-// (208 MB) 0.853 -> 0.786, 48 stacks of 64 x 128 x 128 (252 MB) 0.884 -> 0.777;
-// 256 x 512 x 512 (277 MB) 1.079 -> 1.058; 24 uneven stacks in one graph
-// (156 MB) 0.96 -> 0.87.  Small spectra stay streaming:
-// 64 x 256 x 256 (19 MB) 0.1195 -> 0.129.
+// (208 MB) 0.853 -> 0.786, 48 stacks of 64 x 128 x 128 (252 MB) 0.884 -> 0.777; 24
+// uneven stacks in one graph (156 MB) 0.96 -> 0.87.  At the lower edge: 36 MB
+// 0.188 -> 0.175 (64 x 256 x 512) and 38 MB 0.187 -> 0.168 (128 x 256 x 256); 27 MB
+// would still gain (0.162 -> 0.148 at 64 x 256 x 384), 19 MB loses (0.119 -> 0.128 at
+// 64 x 256 x 256).  At the upper edge 285 MB would gain 2 to 4% (1.091 -> 1.064 at
+// 256 x 512 x 512), 314 MB and more lose 1 to 2% (96 x 1024 x 768, 192 x 512 x 810).
+// Engines side by side, whose spectra together exceed the cache, lose nothing by
+// it (iterations of 8 of 71 MB on 4 streams 2.14 -> 2.12, 16 of 36 MB on 16 2.25 ->
+// 2.13, 4 of 138 MB on 2 2.09 -> 2.04).
 constexpr bool spec_cached(size_t bytes) { return bytes >= (32UL << 20) && bytes <= (256UL << 20); }
 
 // R2C along x of row pairs with the prediction fused in; writes S.  Rows

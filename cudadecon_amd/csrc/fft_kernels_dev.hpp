@@ -280,8 +280,10 @@ template <int N, int COLS = 0> struct CCfg {
 // touching memory, so skipping rows needs no branches.  The inverse y pass
 // with a branch per skipped row needs 75 registers at 1024 points, which
 // leaves one workgroup per CU instead of two (0.393 ms, every row read 0.382,
-// this form 0.357).  Registers of the y transforms: 64 to 2048 points 60-92
-// -> 56-81, of the z filters 92-142 -> 84-126 at 64 to 192 points.
+// this form 0.357).  Registers of the y transforms: 93 -> 77 at 96 points, 85 ->
+// 79 at 192, 62 -> 56 to 61 at 128, 512 and 1024, 124 -> 120 at 810, the same
+// 60 at 2048; of the averaged-table z filters 101 -> 88, 142 -> 126, 92 -> 84
+// and 121 -> 115 at 64, 96, 128 and 192 points.
 // The range check is the vector offset's alone: the scalar offset is defined as
 // taking no part in it (and where it did, a length less a larger scalar offset
 // would be no bound).  So whatever must not be touched has kNoRow, the largest

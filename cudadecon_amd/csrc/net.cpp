@@ -9,8 +9,9 @@
 namespace cdn {
 namespace {
 
-// weight-gradient partial rows, one per workgroup: two or more workgroups per
-// CU, and a quarter of that where a row is 4 times as long (32 <-> 64 channels)
+// weight-gradient partial rows, one per workgroup: two workgroups per CU, and
+// one between 32 and 64 channels, where a row is 4 times as long (the reduction
+// reads 4 bytes a row and weight) and the staged rows take 69 and 97 KB of LDS
 constexpr int WG_CHUNKS = 512;
 constexpr int wg_chunks(int l) { return NET_CIN[l] * NET_COUT[l] > 1024 ? WG_CHUNKS / 2 : WG_CHUNKS; }
 constexpr int WG_CHUNKS_IN1 = 1024;  // first layer

@@ -1175,7 +1175,7 @@ __global__ __launch_bounds__(256) void k_wgrad_in1(const float* __restrict__ raw
 
 // out[c] = sum_g part[g][c] in double, in a fixed order: a workgroup takes 64
 // columns, its 16 waves sum every 16th row each (one thread per column over all
-// rows: 45 us on average over a backward pass with 64 to 512 rows, now 10 with
+// rows: 45 us on average over a backward pass with 64 to 512 rows, now 14 with
 // 256 to 1024).
 constexpr int RED_WAVES = 16;
 __global__ __launch_bounds__(64 * RED_WAVES) void k_reduce_rows(const float* __restrict__ part, int rows, long cols,
